@@ -657,6 +657,16 @@ bool run_groups(Runtime &r, int G, const Pieces &up, const Pieces &down,
     return sync(ds);
 }
 
+// Workspace for the flash partials of a host-pointer SDPA launch on nh heads.
+size_t sdpa_scratch_bytes(int nh, int S_q, int S_kv, int D, int mode)
+{
+    const AttnMode am = mode == ANIMA_HIP_BF16    ? kAttnBF16
+                        : mode == ANIMA_HIP_F32X3 ? kAttnF32X3
+                                                  : kAttnF32;
+    return std::max(flash_split_bytes(nh, S_q, S_kv, D),
+                    attention_balance_bytes(1, S_q, S_kv, nh, D, am));
+}
+
 // Kernels of the host-pointer SDPA for heads [h0, h0 + nh) of the uploaded
 // [BH, S, D] f32 workspace arrays, on stream st: the f32 flash kernel, or the
 // bf16 / f32x3 operand passes (Q and K rows, packed V^T) and their kernel.
@@ -664,7 +674,11 @@ bool sdpa_heads(Runtime &r, int64_t h0, int nh, int S_q, int S_kv, int D, float 
                 int mode, hipStream_t st)
 {
     const bool bf16 = mode == ANIMA_HIP_BF16, x3 = mode == ANIMA_HIP_F32X3;
-    const size_t part_bytes = flash_plan(nh, S_q, S_kv, D).bytes;
+    FlashScratch scr;
+    scr.part = r.scratch.p;
+    scr.part_bytes = flash_split_bytes(nh, S_q, S_kv, D);
+    scr.balance = r.scratch.p;  // a launch uses one of the two
+    scr.balance_bytes = sdpa_scratch_bytes(nh, S_q, S_kv, D, mode);
     FlashProblem p;
     p.q = static_cast<const float *>(r.q.p) + h0 * S_q * D;
     p.k = static_cast<const float *>(r.k.p) + h0 * S_kv * D;
@@ -680,7 +694,7 @@ bool sdpa_heads(Runtime &r, int64_t h0, int nh, int S_q, int S_kv, int D, float 
     p.scale = scale;
     p.causal = causal;
     if (!bf16 && !x3)
-        return launch_flash_f32(p, st, r.scratch.p, part_bytes);
+        return launch_flash_f32(p, st, scr);
     // bf16 copies of Q and K (row kernel without norm/RoPE; rows of [hi | lo]
     // terms in the f32x3 mode) and packed V^T (hi rows, then lo rows).
     const int64_t sp = vt_padded_len(S_kv), w = x3 ? 2 : 1;
@@ -718,12 +732,11 @@ bool sdpa_heads(Runtime &r, int64_t h0, int nh, int S_q, int S_kv, int D, float 
     p.qs = c.os;
     p.ks = ck.os;
     p.vs = vts;
-    return x3 ? launch_flash_x3(p, st, r.scratch.p, part_bytes)
-              : launch_flash_bf16(p, st, r.scratch.p, part_bytes);
+    return x3 ? launch_flash_x3(p, st, scr) : launch_flash_bf16(p, st, scr);
 }
 
 // Head groups of a host-pointer SDPA: the most groups (4 or 2) that still
-// fill the GPU each (flash_plan keeps 8-wave workgroups and no key split)
+// fill the GPU each
 // when the copies are large, else one.  Group g+1 uploads while group g
 // computes, and group g's output comes back while later groups upload.
 int sdpa_groups(int BH, int S_q, int S_kv, int D)
@@ -734,8 +747,7 @@ int sdpa_groups(int BH, int S_q, int S_kv, int D)
     for (int G = Runtime::kMaxGroups; G > 1; G /= 2) {
         if (BH % G != 0)
             continue;
-        const FlashPlan part = flash_plan(BH / G, S_q, S_kv, D);
-        if (part.waves == 8 && part.splits == 1)
+        if (flash_fills_gpu(BH / G, S_q, D))
             return G;
     }
     return 1;
@@ -760,7 +772,7 @@ bool host_sdpa(const float *Q, const float *K, const float *V, float *out, int B
     const int G = sdpa_groups(BH, S_q, S_kv, D), nh = BH / G;
     if (!r.q.reserve(f32_bytes(nq), "workspace Q") || !r.o.reserve(f32_bytes(nq), "workspace O") ||
         !r.k.reserve(f32_bytes(nk), "workspace K") || !r.v.reserve(f32_bytes(nk), "workspace V") ||
-        !r.scratch.reserve(flash_plan(nh, S_q, S_kv, D).bytes, "workspace split-KV partials"))
+        !r.scratch.reserve(sdpa_scratch_bytes(nh, S_q, S_kv, D, mode), "workspace partials"))
         return false;
     if (bf16 || x3) {
         const int64_t w = x3 ? 2 : 1;
@@ -1278,7 +1290,7 @@ bool anima_hip_flash_f32_rawq_dev(const float *q, const float *q_norm_w, float e
     p.D = D;
     p.scale = scale;
     p.causal = is_causal;
-    return launch_flash_f32(p, pick_stream(stream), nullptr, 0);
+    return launch_flash_f32(p, pick_stream(stream));
 }
 
 bool anima_hip_flash_x3_rawq_dev(const float *q, const float *q_norm_w, const float *freqs,
@@ -1508,7 +1520,9 @@ size_t anima_hip_attention_scratch_bytes(int B, int S_q, int Bk, int S_kv, int H
 {
     if (B < 0 || S_q < 0 || Bk < 0 || S_kv < 0 || H < 0 || D < 0)
         return 0;
-    return attention_scratch_bytes(B, S_q, Bk, S_kv, H, D, size_mode(mode), false);
+    const AttnMode am = size_mode(mode);
+    return attention_scratch_bytes(B, S_q, Bk, S_kv, H, D, am, false) +
+           attention_balance_bytes(B, S_q, S_kv, H, D, am);
 }
 
 namespace {
@@ -1549,7 +1563,8 @@ bool attention_dev_call(const char *name, const float *q, const float *k, const 
     const std::string who(name);
     if (!q || !(out || out_t) || !scratch || (S_kv > 0 && (!k || !v)))
         return fail(who + ": null pointer");
-    if (scratch_bytes < attention_scratch_bytes(B, S_q, Bk, S_kv, H, D, am, false))
+    const size_t required = attention_scratch_bytes(B, S_q, Bk, S_kv, H, D, am, false);
+    if (scratch_bytes < required)
         return fail(who + ": scratch smaller than anima_hip_attention_scratch_bytes()");
     AttnInputs in;
     in.q = q;
@@ -1570,6 +1585,7 @@ bool attention_dev_call(const char *name, const float *q, const float *k, const 
     in.D = D;
     in.eps = eps;
     in.mode = am;
+    use_balance_scratch(in, scratch, scratch_bytes, required);
     return run_attention(in, scratch, pick_stream(stream));
 }
 }  // namespace
@@ -1623,12 +1639,12 @@ bool anima_hip_attention(const float *q, const float *k, const float *v, const f
     const int64_t bytes = 2 * f32_bytes(nq) + 2 * f32_bytes(nk);
     int G = 1;
     for (int c = Runtime::kMaxGroups; c > 1 && G == 1 && bytes >= (int64_t(64) << 20); c /= 2) {
-        const FlashPlan part = flash_plan(int64_t(B / c) * H, S_q, S_kv, D);
-        if (B % c == 0 && part.waves == 8 && part.splits == 1)
+        if (B % c == 0 && flash_fills_gpu(int64_t(B / c) * H, S_q, D))
             G = c;
     }
     const int Bg = B / G;
-    const size_t scratch = attention_scratch_bytes(Bg, S_q, Bg, S_kv, H, D, am, false);
+    const size_t required = attention_scratch_bytes(Bg, S_q, Bg, S_kv, H, D, am, false);
+    const size_t scratch = required + attention_balance_bytes(Bg, S_q, S_kv, H, D, am);
     if (!r.q.reserve(f32_bytes(nq), "workspace q") || !r.k.reserve(f32_bytes(nk), "workspace k") ||
         !r.v.reserve(f32_bytes(nk), "workspace v") || !r.o.reserve(f32_bytes(nq), "workspace o") ||
         !r.scratch.reserve(scratch, "workspace scratch"))
@@ -1663,6 +1679,7 @@ bool anima_hip_attention(const float *q, const float *k, const float *v, const f
             in.k = kd + g * gk;
             in.v = vd + g * gk;
             in.out = od + g * gq;
+            use_balance_scratch(in, r.scratch.p, scratch, required);
             return run_attention(in, r.scratch.p, s);
         }))
         return false;
@@ -1836,8 +1853,9 @@ size_t anima_hip_cross_attention_scratch_bytes(const anima_hip_ctx_kv *kv, int B
 {
     if (!kv || B < 0 || S_q < 0)
         return 0;
-    return attention_scratch_bytes(B, S_q, kv->Bc, kv->S_kv, kv->H, kv->D, AttnMode(kv->mode),
-                                   true);
+    const AttnMode am = AttnMode(kv->mode);
+    return attention_scratch_bytes(B, S_q, kv->Bc, kv->S_kv, kv->H, kv->D, am, true) +
+           attention_balance_bytes(B, S_q, kv->S_kv, kv->H, kv->D, am);
 }
 
 namespace {
@@ -1861,7 +1879,9 @@ bool cross_dev_call(const char *name, const float *q, const float *q_norm_w,
     if (!q || !(out || out_t) || !scratch)
         return fail(who + ": null pointer");
     const AttnMode am = AttnMode(kv->mode);
-    if (scratch_bytes < attention_scratch_bytes(B, S_q, kv->Bc, kv->S_kv, kv->H, kv->D, am, true))
+    const size_t required =
+        attention_scratch_bytes(B, S_q, kv->Bc, kv->S_kv, kv->H, kv->D, am, true);
+    if (scratch_bytes < required)
         return fail(who + ": scratch smaller than anima_hip_cross_attention_scratch_bytes()");
     AttnInputs in;
     in.q = q;
@@ -1880,6 +1900,7 @@ bool cross_dev_call(const char *name, const float *q, const float *q_norm_w,
     in.D = kv->D;
     in.eps = eps;
     in.mode = am;
+    use_balance_scratch(in, scratch, scratch_bytes, required);
     return run_attention(in, scratch, pick_stream(stream));
 }
 }  // namespace
@@ -1930,13 +1951,13 @@ bool anima_hip_cross_attention(const float *q, const float *q_norm_w, const anim
     int G = 1;
     for (int c = Runtime::kMaxGroups; c > 1 && G == 1 && 2 * f32_bytes(nq) >= (size_t(64) << 20);
          c /= 2) {
-        const FlashPlan part = flash_plan(int64_t(B / c) * kv->H, S_q, kv->S_kv, kv->D);
-        if (B % c == 0 && part.waves == 8 && part.splits == 1)
+        if (B % c == 0 && flash_fills_gpu(int64_t(B / c) * kv->H, S_q, kv->D))
             G = c;
     }
     const int Bg = B / G, Bkg = kv->Bc == 1 ? 1 : Bg;
-    const size_t scratch =
+    const size_t required =
         attention_scratch_bytes(Bg, S_q, Bkg, kv->S_kv, kv->H, kv->D, am, true);
+    const size_t scratch = required + attention_balance_bytes(Bg, S_q, kv->S_kv, kv->H, kv->D, am);
     const float *qw = nullptr;
     if (!r.q.reserve(f32_bytes(nq), "workspace q") || !r.o.reserve(f32_bytes(nq), "workspace o") ||
         !r.scratch.reserve(scratch, "workspace scratch"))
@@ -1971,6 +1992,7 @@ bool anima_hip_cross_attention(const float *q, const float *q_norm_w, const anim
             in.D = kv->D;
             in.eps = eps;
             in.mode = am;
+            use_balance_scratch(in, r.scratch.p, scratch, required);
             return run_attention(in, r.scratch.p, s);
         }))
         return false;

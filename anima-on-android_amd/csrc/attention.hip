@@ -66,7 +66,27 @@ size_t attention_scratch_bytes(int B, int S_q, int Bk, int S_kv, int H, int D, A
         if (mode != kAttnF32)
             n += round_up(prepared_v_bytes(Bk, S_kv, H, D, mode));
     }
-    return n + round_up(flash_plan(int64_t(B) * H, S_q, S_kv, D).bytes);
+    return n + round_up(flash_split_bytes(int64_t(B) * H, S_q, S_kv, D));
+}
+
+namespace {
+const FlashTimes &times_of(AttnMode mode)
+{
+    return mode == kAttnBF16 ? kTimesBF16 : mode == kAttnF32X3 ? kTimesX3 : kTimesF32;
+}
+}  // namespace
+
+size_t attention_balance_bytes(int B, int S_q, int S_kv, int H, int D, AttnMode mode)
+{
+    return round_up(flash_balance_bytes(int64_t(B) * H, S_q, S_kv, D, times_of(mode)));
+}
+
+void use_balance_scratch(AttnInputs &in, void *scratch, size_t scratch_bytes, size_t required)
+{
+    if (scratch_bytes <= required)
+        return;
+    in.balance = static_cast<char *>(scratch) + required;
+    in.balance_bytes = scratch_bytes - required;
 }
 
 namespace {
@@ -198,9 +218,14 @@ bool run_attention(const AttnInputs &in, void *scratch, hipStream_t st)
         if (mode != kAttnF32)
             cur += round_up(prepared_v_bytes(in.Bk, S_kv, H, D, mode));
     }
-    // Split-KV partials (small problems only).
-    void *part = cur;
-    const size_t part_bytes = flash_plan(int64_t(B) * H, S_q, S_kv, D).bytes;
+    // Partials: of a split grid (small problems only), of a balanced grid.
+    FlashScratch scr;
+    scr.part = cur;
+    scr.part_bytes = flash_split_bytes(int64_t(B) * H, S_q, S_kv, D);
+    if (in.balance && (reinterpret_cast<uintptr_t>(in.balance) & 15u) == 0) {
+        scr.balance = in.balance;
+        scr.balance_bytes = in.balance_bytes;
+    }
 
     // Cross-attention (K/V prepared, no RoPE) in f32x3 on a grid of at least
     // one 8-wave workgroup per CU: the flash kernel prepares its own query
@@ -219,11 +244,12 @@ bool run_attention(const AttnInputs &in, void *scratch, hipStream_t st)
     // 8-wave workgroup per CU it measured the same as the row pass (4096 x
     // 512, B = 2: 65.7 against 65.9 us, bit-identical).
     const auto a16 = [](const void *x) { return (reinterpret_cast<uintptr_t>(x) & 15u) == 0; };
-    const FlashPlan raw_plan = flash_plan(int64_t(B) * H, S_q, S_kv, D,
-                                          mode == kAttnF32X3 ? kTileUsX3 : kTileUsF32);
+    // A dealt workgroup of a balanced grid repeats it for its second part, as
+    // it repeats the query load.
+    const FlashPlan raw_plan = flash_plan(int64_t(B) * H, S_q, S_kv, D, times_of(mode), false,
+                                          scr.part_bytes, scr.balance_bytes);
     const bool raw_kernel =
-        mode == kAttnBF16 ? flash_bf16_raw_q(int64_t(B) * H, S_q, S_kv)
-                          : raw_plan.waves == 8 && raw_plan.splits == 1;
+        mode == kAttnBF16 ? flash_bf16_raw_q(raw_plan, S_kv) : raw_plan.waves == 8;
     const bool raw_q = !q_ready && prepared && !in.freqs && D == 128 && a16(in.q) &&
                        ld_q % 4 == 0 && (!in.q_norm_w || a16(in.q_norm_w)) && raw_kernel;
 
@@ -272,11 +298,11 @@ bool run_attention(const AttnInputs &in, void *scratch, hipStream_t st)
     }
     switch (mode) {
     case kAttnBF16:
-        return launch_flash_bf16(p, st, part, part_bytes);
+        return launch_flash_bf16(p, st, scr);
     case kAttnF32X3:
-        return launch_flash_x3(p, st, part, part_bytes);
+        return launch_flash_x3(p, st, scr);
     default:
-        return launch_flash_f32(p, st, part, part_bytes);
+        return launch_flash_f32(p, st, scr);
     }
 }
 

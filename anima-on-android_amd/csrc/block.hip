@@ -226,9 +226,10 @@ __global__ __launch_bounds__(256) void gate_residual_kernel(ResidualArgs a)
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// Scratch regions of one sub-block, 256-byte aligned, in order.
+// Scratch regions of one sub-block, 256-byte aligned, in order: what it needs
+// (`required`), then what a balanced flash grid can use beside that.
 struct BlockScratch {
-    size_t terms, q, k, v, o, y, attn, lin, total;
+    size_t terms, q, k, v, o, y, attn, lin, required, total;
 };
 
 BlockScratch block_scratch(int B, int S, int Dm, int H, int D, int Bk, int S_kv, AttnMode mode,
@@ -245,7 +246,8 @@ BlockScratch block_scratch(int B, int S, int Dm, int H, int D, int Bk, int S_kv,
     s.y = round_up256(M * size_t(Dm) * 4);
     s.attn = round_up256(attention_scratch_bytes(B, S, Bk, S_kv, H, D, mode, cross));
     s.lin = round_up256(linear_scratch_bytes(int(M), int(HD), !bf16));
-    s.total = s.terms + s.q + s.k + s.v + s.o + s.y + s.attn + s.lin;
+    s.required = s.terms + s.q + s.k + s.v + s.o + s.y + s.attn + s.lin;
+    s.total = s.required + attention_balance_bytes(B, S, S_kv, H, D, mode);
     return s;
 }
 
@@ -349,7 +351,7 @@ bool run_attention_block(const BlockProblem &p, void *scratch, size_t scratch_by
         return fail("attention_block: null pointer");
     const BlockScratch s = block_scratch(B, S, Dm, H, D, cross ? p.Bk : B, cross ? p.S_kv : S,
                                          p.mode, cross);
-    if (!scratch || scratch_bytes < s.total || !aligned16(scratch))
+    if (!scratch || scratch_bytes < s.required || !aligned16(scratch))
         return fail("attention_block: scratch smaller than the size query or not 16-byte aligned");
     char *cur = static_cast<char *>(scratch);
     auto take = [&](size_t n) {
@@ -413,6 +415,7 @@ bool run_attention_block(const BlockProblem &p, void *scratch, size_t scratch_by
         in.ld_t = kp;
         in.lo_t = bf16 ? 0 : int64_t(hi_bytes / 2);
     }
+    use_balance_scratch(in, scratch, scratch_bytes, s.required);
     if (!run_attention(in, attn, st))
         return false;
 

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include "flash_deal.h"
 #include <cstdint>
 #include <string>
 
@@ -61,53 +62,92 @@ struct FlashProblem {
 };
 bool term_out_ok(const TermOut &t);  // alignment of a set term output
 
-// Launch shape of the D == 128 flash kernels.  A grid of B*H*ceil(S_q/256)
-// workgroups of 8 waves fills the GPU when it has at least one workgroup per
-// CU.  Smaller problems (short sequences, few heads) use workgroups of 4
-// waves and, when the caller provides scratch, split the key range over
-// `splits` workgroups per query tile ("split-KV"): split s takes key tiles
-// [s*tiles, (s+1)*tiles) (64 keys each) and writes its output normalised by
-// its own row sum, plus that row's (max, sum), to scratch; flash_combine
-// merges the splits into O.
+// Launch shape of the D == 128 flash kernels: T = B*H*ceil(S_q/256) query
+// tiles of 8-wave workgroups, or twice as many of 4 waves, over n key tiles of
+// 64 keys, on 256 CUs that hold one workgroup each.  Four shapes:
+//   whole     8-wave workgroups, one query tile each;
+//   small     4-wave workgroups, one query tile each (T < 256);
+//   split     4-wave workgroups, the key range of every query tile split over
+//             `splits` of them ("split-KV"): split s takes key tiles
+//             [s*tiles, (s+1)*tiles);
+//   balanced  the largest multiple of 256 query tiles whole, and the key tiles
+//             of the `ntail` others as one list dealt out evenly, `u` to each
+//             of the last workgroups (T = 288 over 36 key tiles: 36 + 5 tiles
+// A workgroup that sees part of a query tile's keys writes its output
+// normalised by its own row sum, plus that row's (max, sum), to scratch, and
+// flash_combine merges the parts into O.
 struct FlashPlan {
     int waves = 8;
     int splits = 1;
     int tiles = 1 << 30;  // key tiles per split
-    size_t bytes = 0;     // scratch for the partials (0 when unsplit)
+    int full = 0;         // balanced: query tiles run whole
+    int ntail = 0;        // balanced: query tiles dealt out
+    int nk = 0;           // balanced: key tiles of a query tile
+    int u = 0;            // balanced: key tiles per workgroup (0: another shape)
+    size_t bytes = 0;     // scratch for the partials (0 when every tile runs whole)
 };
-// tile_us > 0: the kernel's time per 64-key tile in a 4-wave workgroup (us);
-// the key range is then split only where the tiles a workgroup no longer
-// walks are worth more than a split grid's fixed cost (kSplitCostUs: every
-// split loads its query tile and writes f32 partials that the combine pass
-// reads back).  tile_us == 0 always splits a small grid: the scratch size
-// every mode's plan fits in.
-FlashPlan flash_plan(int64_t BH, int S_q, int S_kv, int D, float tile_us = 0.0f);
-// Measured on MI355X at 32 heads x 256 queries (unsplit 4-wave grids over
-// 4 and 8 key tiles; split grids against them, combine included).
-constexpr float kSplitCostUs = 13.0f;
-constexpr float kTileUsF32 = 9.1f, kTileUsBF16 = 1.3f, kTileUsX3 = 2.5f;
+// What a kernel takes per 64-key tile (us) in a 4-wave and in an 8-wave
+// workgroup when every CU holds one, measured on MI355X (4-wave: 32 heads x
+// 256 queries, unsplit grids over 4 and 8 key tiles; 8-wave: 32 heads x 4096
+// queries and keys).  The bf16-MFMA kernels are bound by power: an 8-wave
+// round of at most about 0.7 of the CUs clocks higher, down to `part` of w8
+// (x3, T = 288 .. 800: 0.66 .. 0.76 of the full rounds' time per tile); the
+// f32 MFMA runs at full clock either way.
+struct FlashTimes {
+    float w4, w8, part;
+};
+constexpr FlashTimes kTimesF32{9.1f, 15.7f, 1.0f}, kTimesBF16{1.3f, 1.9f, 0.7f},
+    kTimesX3{2.5f, 4.6f, 0.7f};
+// Fixed cost (us) of split grids and of balanced ones, whose parts are twice
+// as tall: every part loads its query tile and writes f32 partials, which the
+// combine pass reads back (25 to 31 us at T = 144 and 288, every mode).
+constexpr float kSplitCostUs = 13.0f, kBalanceCostUs = 27.0f;
+// The shape with the least predicted time among those whose partials fit:
+// part_bytes of scratch for `split`, balance_bytes for `balanced` (causal
+// calls, whose tiles differ in length, are not balanced).
+FlashPlan flash_plan(int64_t BH, int S_q, int S_kv, int D, const FlashTimes &t, bool causal,
+                     size_t part_bytes, size_t balance_bytes);
+// Scratch that holds the partials of a split grid in every mode, and that of
+// a balanced grid (0 where none would run).
+size_t flash_split_bytes(int64_t BH, int S_q, int S_kv, int D);
+size_t flash_balance_bytes(int64_t BH, int S_q, int S_kv, int D, const FlashTimes &t);
+constexpr size_t kMaxFlashBalanceBytes = size_t(511) * 256 * (128 * 4 + 8);  // 65 MiB
+// A grid of 8-wave workgroups with at least one for each CU.
+bool flash_fills_gpu(int64_t BH, int S_q, int D);
 
-// What a split workgroup writes (device view).  Partials are laid out
-// [splits][BH][S_q][128] f32 and (max, sum) pairs [splits][BH][S_q] float2,
-// the max in log2 units of the scaled scores.
+// Scratch a flash launch may use, 16-byte aligned; either may be null.
+struct FlashScratch {
+    void *part = nullptr;
+    size_t part_bytes = 0;
+    void *balance = nullptr;
+    size_t balance_bytes = 0;
+};
+
+// What a workgroup that sees part of the keys writes (device view).  Partials
+// of a split grid are laid out [splits][BH][S_q][128] f32 and (max, sum) pairs
+// [splits][BH][S_q] float2; those of a balanced grid by slots of 256 rows,
+// slot t + g for tail tile t and share g (along the list either t or g rises
+// by one from part to part).  The max is in log2 units of the scaled scores.
 struct FlashSplitArgs {
     int n = 1;
     int tiles = 1 << 30;
+    int full = 0, ntail = 0, nk = 1, u = 0;
+    int ng = 0;        // balanced: shares
+    int nshorter = 0;  // balanced: workgroups that take a shorter piece
     int64_t BH = 0;
     float *part = nullptr;
     float2 *ml = nullptr;
 };
-// Split descriptor for plan `pl` over scratch `part` (nullptr or too small:
-// unsplit).
-FlashSplitArgs flash_split_args(const FlashPlan &pl, int64_t BH, int S_q, void *part,
-                                size_t part_bytes);
+struct FlashWhole {};  // in FlashDeal's place where no query tile is dealt out
+FlashSplitArgs flash_split_args(const FlashPlan &pl, int64_t BH, int S_q, const FlashScratch &s,
+                                FlashDeal &deal);
+// Workgroups of the launch: BM query rows per tile.
+int64_t flash_blocks(const FlashSplitArgs &sa, int64_t BH, int S_q, int BM);
 // O[b,h,q,:] = sum_s w_s P_s[bh,q,:] / sum_s w_s, w_s = l_s * 2^(m_s - max_s m_s).
 bool launch_flash_combine(const FlashProblem &p, const FlashSplitArgs &sa, hipStream_t st);
 
 // f32 inputs, f32 MFMA (D == 128) or the generic kernel (any D <= 1024).
-// `part` is optional split-KV scratch of flash_plan(...).bytes.
-bool launch_flash_f32(const FlashProblem &p, hipStream_t st, void *part = nullptr,
-                      size_t part_bytes = 0);
+bool launch_flash_f32(const FlashProblem &p, hipStream_t st, const FlashScratch &scr = {});
 // True when launch_flash_f32 would take the MFMA path for this problem.
 bool flash_f32_fast_path(const FlashProblem &p);
 
@@ -115,13 +155,12 @@ bool flash_f32_fast_path(const FlashProblem &p);
 // bf16 MFMA with f32 accumulation and f32 softmax; D == 128 and scale > 0.
 // `v` points at the packed V^T and `vs` holds its {batch, head, d-row}
 // strides (the d-row stride is vt_padded_len(S_kv)).
-bool launch_flash_bf16(const FlashProblem &p, hipStream_t st, void *part = nullptr,
-                       size_t part_bytes = 0);
-// True when launch_flash_bf16 runs this shape as two 4-wave workgroups per CU
+bool launch_flash_bf16(const FlashProblem &p, hipStream_t st, const FlashScratch &scr = {});
+// True when launch_flash_bf16 runs plan `pl` as two 4-wave workgroups per CU
 // (large grids over short key ranges), where the kernel also takes raw query
 // rows (FlashProblem::rq) at no cost: their larger load overlaps the other
 // workgroup's tiles.
-bool flash_bf16_raw_q(int64_t BH, int S_q, int S_kv);
+bool flash_bf16_raw_q(const FlashPlan &pl, int S_kv);
 
 // V^T layout of the bf16 path: per (batch, head) a [D][Sp] bf16 matrix with
 // Sp = vt_padded_len(S_kv), zero beyond S_kv, and within every group of 16
@@ -146,8 +185,7 @@ bool launch_vt_pack(const float *v, Strides vs, uint16_t *vt, Strides vts, int B
 // through qs/ks (row starts); v: packed term V^T, per (batch, head) the D hi
 // rows then the D lo rows of the V^T layout above, strides {batch, head,
 // d-row = vt_padded_len(S_kv)}.  D == 128, scale > 0.
-bool launch_flash_x3(const FlashProblem &p, hipStream_t st, void *part = nullptr,
-                     size_t part_bytes = 0);
+bool launch_flash_x3(const FlashProblem &p, hipStream_t st, const FlashScratch &scr = {});
 // Pack V (f32 view as for launch_vt_pack) into the term V^T layout above.
 bool launch_vt_pack_terms(const float *v, Strides vs, uint16_t *vt, Strides vts, int B, int H,
                           int S_kv, int D, hipStream_t st);
@@ -325,6 +363,10 @@ struct AttnInputs {
     // Token-row strides (elements) of q and of the raw k/v: 0 means H*D
     // (dense); wider when they are column blocks of one fused projection.
     int64_t ld_q = 0, ld_kv = 0;
+    // Optional scratch for a balanced flash grid's partials, beside the
+    // required scratch: attention_balance_bytes() of it, 16-byte aligned.
+    void *balance = nullptr;
+    size_t balance_bytes = 0;
 };
 // A self-attention's three operands in one launch (prologue.hip): q and k
 // [B, S, H, 128] f32 with token rows ld elements apart and batch entries
@@ -372,8 +414,14 @@ bool launch_gemm_f32a_qkv(const float *a, int64_t lda, const uint16_t *w, int64_
                           const QkvPrep &p, hipStream_t st);
 size_t prepared_k_bytes(int Bk, int S_kv, int H, int D, AttnMode mode);
 size_t prepared_v_bytes(int Bk, int S_kv, int H, int D, AttnMode mode);
+// Scratch run_attention needs, and what it can use beside that
+// (AttnInputs::balance).  The size queries report their sum; a call with the
+// first alone runs too, without a balanced grid.
 size_t attention_scratch_bytes(int B, int S_q, int Bk, int S_kv, int H, int D, AttnMode mode,
                                bool kv_prepared);
+size_t attention_balance_bytes(int B, int S_q, int S_kv, int H, int D, AttnMode mode);
+// Points in.balance behind the required scratch when scratch_bytes has room.
+void use_balance_scratch(AttnInputs &in, void *scratch, size_t scratch_bytes, size_t required);
 bool prepare_kv(const float *k, const float *v, const float *k_norm_w, const float *freqs,
                 void *k_out, void *v_out, int Bk, int S_kv, int H, int D, float eps,
                 AttnMode mode, hipStream_t st);

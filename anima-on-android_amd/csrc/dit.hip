@@ -537,9 +537,10 @@ SubLayout sub_layout(const anima_hip_dit *d, int B, int64_t S, int kind)
     return l;
 }
 
-// Scratch regions of one forward, 256-byte aligned, in order.
+// Scratch regions of one forward, 256-byte aligned, in order: what it needs
+// (`required`), then what balanced flash grids can use beside that.
 struct DitScratch {
-    size_t x, y, patch, f, arena, total;
+    size_t x, y, patch, f, arena, required, total;
 };
 
 DitScratch dit_scratch(const anima_hip_dit *d, int B, int64_t S)
@@ -558,7 +559,11 @@ DitScratch dit_scratch(const anima_hip_dit *d, int B, int64_t S)
     size_t arena = std::max(self.total, std::max(cross.total, mlp.total));
     arena = std::max(arena, round_up256(size_t(M) * linear_terms_ld(c.dim) * 2) * 2);
     s.arena = round_up256(arena);
-    s.total = s.x + s.y + s.patch + s.f + s.arena;
+    s.required = s.x + s.y + s.patch + s.f + s.arena;
+    const auto balance = [&](int S_kv) {
+        return attention_balance_bytes(B, int(S), S_kv, c.heads, c.head_dim, d->attn);
+    };
+    s.total = s.required + std::max(balance(int(S)), balance(std::max(d->ctx_S, 1)));
     return s;
 }
 
@@ -646,7 +651,8 @@ bool dit_project_terms(const anima_hip_dit *d, const uint16_t *t, int K, const u
 bool dit_sublayer(const anima_hip_dit *d, const BlockWeights &bw, int kind, float *x,
                   const float *mod, const float *pend_y, int pend_parts, const float *pend_mod,
                   float *y, size_t y_bytes, int *y_parts, int B,
-                  int64_t S, const float *freqs, void *arena, hipStream_t st)
+                  int64_t S, const float *freqs, void *arena, void *balance,
+                  size_t balance_bytes, hipStream_t st)
 {
     const anima_hip_dit_config &c = d->cfg;
     const int D = c.dim, HD = c.heads * c.head_dim;
@@ -732,6 +738,8 @@ bool dit_sublayer(const anima_hip_dit *d, const BlockWeights &bw, int kind, floa
     in.eps = 1e-6f;
     in.mode = d->attn;
     in.out = o;
+    in.balance = balance;
+    in.balance_bytes = balance_bytes;
     if (fused_qkv) {
         if (!launch_gemm_f32a_qkv(reinterpret_cast<const float *>(terms), D, bw.w_qkv, d->ld_d, D,
                                   qp, st))
@@ -805,7 +813,7 @@ bool dit_run(anima_hip_dit *d, const float *x, int64_t xb, const float *sigma, i
     if (M > INT32_MAX / 8)
         return fail("dit: too many tokens");
     const DitScratch s = dit_scratch(d, B, S);
-    if (!scratch || scratch_bytes < s.total || !aligned16(scratch))
+    if (!scratch || scratch_bytes < s.required || !aligned16(scratch))
         return fail("dit: scratch smaller than anima_hip_dit_scratch_bytes() or not 16-byte "
                     "aligned");
     char *base = static_cast<char *>(scratch);
@@ -878,7 +886,8 @@ bool dit_run(anima_hip_dit *d, const float *x, int64_t xb, const float *sigma, i
             const float *mod = d->mods + (3 * i + kind) * mod_stride;
             int parts = 1;
             if (!dit_sublayer(d, d->blk[i], kind, xr, mod, pend_mod ? yp : nullptr, pend_parts,
-                              pend_mod, yp, s.y, &parts, B, S, freqs, arena, st))
+                              pend_mod, yp, s.y, &parts, B, S, freqs, arena, base + s.required,
+                              scratch_bytes - s.required, st))
                 return false;
             pend_mod = mod;
             pend_parts = parts;

@@ -50,8 +50,8 @@ struct F32Args {
     int H, S_q, S_kv, n_qtiles;
     float c;     // scale * log2(e)
     int causal;
-    FlashSplitArgs split;  // n == 1: write O; n > 1: write this split's partial
-    TermOut ot;            // n == 1 and ot.t set: O as bf16 terms
+    FlashSplitArgs split;  // which parts this workgroup computes
+    TermOut ot;            // whole tiles, ot.t set: O as bf16 terms
     // q holds raw projection rows (RawQ, no RoPE): the kernel applies the
     // per-head RMSNorm (weight qw, optional) itself.
     int raw_q;
@@ -116,8 +116,8 @@ __device__ __forceinline__ int acc_row(int r, int h)
     return 8 * (r >> 2) + 4 * h + (r & 3);
 }
 
-template <int NW>
-__global__ __launch_bounds__(NW * 64, 1) void flash_f32_d128(F32Args a)
+template <int NW, typename Deal>
+__global__ __launch_bounds__(NW * 64, 1) void flash_f32_d128(F32Args a, Deal deal)
 {
     constexpr int NT = NW * 64;
     constexpr int BM = NW * 32;
@@ -138,13 +138,13 @@ __global__ __launch_bounds__(NW * 64, 1) void flash_f32_d128(F32Args a)
     // and read its K/V through that XCD's L2 (the dispatcher's round-robin
     // order had every XCD fetch every head's K/V: 1.21 GB per launch at
     // 4096 tokens, B = 2, against 268 MB of algorithmic bytes).
-    const int blk = flash_tile::xcd_major_block();
-    const int sp = blk % a.split.n;
-    const int qt = (blk / a.split.n) % a.n_qtiles;
-    const int bh = (blk / a.split.n) / a.n_qtiles;
+    const flash_tile::FlashWork work(a.split, deal, a.n_qtiles, a.S_q, BM);
+    if (work.jn == 0)
+        return;
+    const int bh = work.bh;
     const int b = bh / a.H;
     const int h = bh - b * a.H;
-    const int q_tile0 = qt * BM;
+    const int q_tile0 = work.qt * BM;
     const int qrow = q_tile0 + wave * 32 + col;
 
     const float *qp = a.q + b * a.qb + h * a.qh;
@@ -180,9 +180,9 @@ __global__ __launch_bounds__(NW * 64, 1) void flash_f32_d128(F32Args a)
         const int last_row = min(a.S_q, q_tile0 + BM);
         kv_end = min(kv_end, last_row);
     }
-    // Key tiles [j0, j1) of this split (all of them when unsplit).
-    const int j0 = sp * a.split.tiles;
-    const int j1 = min((kv_end + kBN - 1) / kBN, j0 + a.split.tiles);
+    // Key tiles [j0, j1) of this part (all of them when unsplit).
+    const int j0 = work.j0;
+    const int j1 = min((kv_end + kBN - 1) / kBN, j0 + work.jn);
 
     // Next-tile staging registers, used for V then for K so only one
     // half-tile is held at a time.
@@ -329,8 +329,8 @@ __global__ __launch_bounds__(NW * 64, 1) void flash_f32_d128(F32Args a)
     if (qrow < a.S_q) {
         float *op = a.o + b * a.ob + h * a.oh + qrow * a.os;
         uint16_t *tp = a.ot.t ? a.ot.t + b * a.ot.tb + h * a.ot.th + qrow * a.ot.ts : nullptr;
-        if (a.split.n > 1) {
-            const int64_t prow = (int64_t(sp) * a.split.BH + bh) * a.S_q + qrow;
+        if (work.prow >= 0) {
+            const int64_t prow = work.prow + wave * 32 + col;
             op = a.split.part + prow * kD;
             tp = nullptr;
             if (half == 0)
@@ -438,16 +438,17 @@ void fill_common(T &g, const FlashProblem &p)
 bool aligned16(const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0; }
 bool stride4(const Strides &s) { return s.b % 4 == 0 && s.h % 4 == 0 && s.s % 4 == 0; }
 
-template <int NW>
-bool launch_d128(const F32Args &a, int64_t BH, hipStream_t st)
+template <int NW, typename Deal>
+bool launch_d128(const F32Args &a, const Deal &deal, int64_t BH, hipStream_t st)
 {
     constexpr int BM = NW * 32;
     F32Args g = a;
     g.n_qtiles = (g.S_q + BM - 1) / BM;
-    const int64_t nblk = BH * g.n_qtiles * g.split.n;
+    const int64_t nblk = flash_blocks(g.split, BH, g.S_q, BM);
     if (nblk > INT32_MAX)
         return fail("flash_f32: problem too large for one launch");
-    hipLaunchKernelGGL(flash_f32_d128<NW>, dim3(unsigned(nblk)), dim3(NW * 64), 0, st, g);
+    hipLaunchKernelGGL((flash_f32_d128<NW, Deal>), dim3(unsigned(nblk)), dim3(NW * 64), 0, st, g,
+                       deal);
     return hip_ok(hipGetLastError(), "flash_f32_d128 launch");
 }
 
@@ -459,7 +460,7 @@ bool flash_f32_fast_path(const FlashProblem &p)
            stride4(p.qs) && stride4(p.ks) && stride4(p.vs) && stride4(p.os);
 }
 
-bool launch_flash_f32(const FlashProblem &p, hipStream_t st, void *part, size_t part_bytes)
+bool launch_flash_f32(const FlashProblem &p, hipStream_t st, const FlashScratch &scr)
 {
     const int64_t BH = int64_t(p.B) * p.H;
     if (BH == 0 || p.S_q == 0)
@@ -485,11 +486,15 @@ bool launch_flash_f32(const FlashProblem &p, hipStream_t st, void *part, size_t 
         a.raw_q = raw_q ? 1 : 0;
         a.qw = p.rq.w;
         a.eps = p.rq.eps;
-        const FlashPlan pl = flash_plan(BH, p.S_q, p.S_kv, p.D, kTileUsF32);
-        a.split = flash_split_args(pl, BH, p.S_q, part, part_bytes);
-        if (!(pl.waves == 4 ? launch_d128<4>(a, BH, st) : launch_d128<8>(a, BH, st)))
+        const FlashPlan pl = flash_plan(BH, p.S_q, p.S_kv, p.D, kTimesF32, p.causal,
+                                        scr.part_bytes, scr.balance_bytes);
+        FlashDeal deal;
+        a.split = flash_split_args(pl, BH, p.S_q, scr, deal);
+        if (!(pl.waves == 4 ? launch_d128<4>(a, FlashWhole{}, BH, st)
+              : pl.u > 0    ? launch_d128<8>(a, deal, BH, st)
+                            : launch_d128<8>(a, FlashWhole{}, BH, st)))
             return false;
-        return a.split.n == 1 || launch_flash_combine(p, a.split, st);
+        return (a.split.n == 1 && a.split.u == 0) || launch_flash_combine(p, a.split, st);
     }
     if (p.D > 1024)
         return fail("flash_f32: head dim " + std::to_string(p.D) + " > 1024 is not supported");

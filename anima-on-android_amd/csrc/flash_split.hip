@@ -1,6 +1,6 @@
-// Split-KV support of the D == 128 flash kernels: the launch plan for
-// problems too small to fill the GPU, and the kernel that merges the
-// per-split partial outputs.
+// Launch plans of the D == 128 flash kernels (which query tiles run whole and
+// whose keys are shared out over several workgroups) and the kernel that
+// merges the partial outputs.
 //
 // Merging follows from the online-softmax identity the flash kernels already
 // use between key tiles (anima_rt/include/cpu/flash_attention.h:145-178 rescales
@@ -10,6 +10,7 @@
 #include "common.h"
 #include "flash_tile.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace anima_hip {
@@ -19,7 +20,9 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kD = 128;
 constexpr int kBN = 64;            // keys per tile of the flash kernels
-constexpr int kTargetBlocks = 256; // one flash workgroup per CU of an MI355X (256 CUs)
+constexpr int kTargetBlocks = kFlashTargetBlocks;
+constexpr int kBM8 = 256;          // query rows of an 8-wave workgroup
+constexpr size_t kSlotBytes = size_t(kBM8) * (kD * sizeof(float) + sizeof(float2));
 
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 size_t round_up256(size_t n) { return (n + 255) / 256 * 256; }
@@ -27,30 +30,54 @@ size_t round_up256(size_t n) { return (n + 255) / 256 * 256; }
 struct CombineArgs {
     float *o;
     int64_t ob, oh, os;
-    int H, S_q;
+    int H, S_q, n_qtiles;
     FlashSplitArgs sa;
     TermOut ot;     // set: O as bf16 terms instead of f32 at o
-    int64_t total;  // BH * S_q * 32 float4 columns
+    int64_t total;  // rows * 32 float4 columns
 };
 
-// One thread per (row, float4 of the head dim).
+// One thread per (row, float4 of the head dim).  BAL: the rows are those of a
+// balanced grid's tail tiles, whose parts differ in number.  Bound by the
+// partials' bytes (2304 tokens, B = 2, H = 16: 256 parts of 128 KiB).
+template <bool BAL>
 __global__ __launch_bounds__(256) void flash_combine_kernel(CombineArgs a)
 {
     const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
     if (idx >= a.total)
         return;
-    const int64_t row = idx >> 5;  // bh * S_q + q
+    int64_t row = idx >> 5;  // bh * S_q + q
     const int c4 = int(idx & 31);
-    const int64_t plane = a.sa.BH * a.S_q;
+    // Part s of this row is at partial row row0 + s * plane.
+    int64_t bh, row0, plane;
+    int q, n;
+    if (BAL) {
+        const int t = int(row / kBM8), r = int(row - int64_t(t) * kBM8);
+        const int tile = a.sa.full + t;
+        bh = tile / a.n_qtiles;
+        q = int(tile - bh * a.n_qtiles) * kBM8 + r;
+        const int64_t k0 = int64_t(t) * a.sa.nk;
+        const int g0 = int(k0 / a.sa.u), g1 = int((k0 + a.sa.nk - 1) / a.sa.u);
+        n = g1 - g0 + 1;
+        if (q >= a.S_q)
+            return;
+        row0 = int64_t(t + g0) * kBM8 + r;
+        plane = kBM8;
+    } else {
+        bh = row / a.S_q;
+        q = int(row - bh * a.S_q);
+        n = a.sa.n;
+        row0 = row;
+        plane = a.sa.BH * a.S_q;
+    }
     // Groups of kU splits: all loads of a group are issued before any use,
     // so the merge costs a few memory latencies rather than one per split.
     constexpr int kU = 8;
     float mx = -INFINITY;
-    for (int s0 = 0; s0 < a.sa.n; s0 += kU) {
+    for (int s0 = 0; s0 < n; s0 += kU) {
         float2 v[kU];
 #pragma unroll
         for (int u = 0; u < kU; ++u)
-            v[u] = s0 + u < a.sa.n ? a.sa.ml[(s0 + u) * plane + row] : make_float2(0.f, 0.f);
+            v[u] = s0 + u < n ? a.sa.ml[(s0 + u) * plane + row0] : make_float2(0.f, 0.f);
         // A split with l == 0 saw no key (causal) or only masked or NaN
         // scores; a NaN l (a NaN score among finite ones) joins and makes
         // the row NaN, as in the reference.
@@ -61,13 +88,13 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(CombineArgs a)
     }
     float lsum = 0.0f;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < a.sa.n; s0 += kU) {
+    for (int s0 = 0; s0 < n; s0 += kU) {
         float2 v[kU];
         f32x4 x[kU];
 #pragma unroll
         for (int u = 0; u < kU; ++u) {
-            const bool in = s0 + u < a.sa.n;
-            const int64_t prow = (s0 + u) * plane + row;
+            const bool in = s0 + u < n;
+            const int64_t prow = (s0 + u) * plane + row0;
             v[u] = in ? a.sa.ml[prow] : make_float2(0.f, 0.f);
             x[u] = in ? *reinterpret_cast<const f32x4 *>(a.sa.part + prow * kD + 4 * c4)
                       : f32x4{0.f, 0.f, 0.f, 0.f};
@@ -82,8 +109,6 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(CombineArgs a)
         }
     }
     const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
-    const int64_t bh = row / a.S_q;
-    const int q = int(row - bh * a.S_q);
     const int b = int(bh / a.H), h = int(bh - int64_t(b) * a.H);
     flash_tile::store_out4(acc * inv, a.o + b * a.ob + h * a.oh + q * a.os,
                            a.ot.t ? a.ot.t + b * a.ot.tb + h * a.ot.th + q * a.ot.ts : nullptr,
@@ -98,10 +123,14 @@ bool term_out_ok(const TermOut &t)
            t.ts % 8 == 0 && t.lo % 8 == 0 && t.lo >= 0;
 }
 
-FlashPlan flash_plan(int64_t BH, int S_q, int S_kv, int D, float tile_us)
+namespace {
+
+// The split shape, which every mode's scratch must hold: 4-wave workgroups,
+// the key range over ~256 of them.
+FlashPlan split_plan(int64_t BH, int S_q, int S_kv, int D)
 {
     FlashPlan pl;
-    if (D != kD || BH <= 0 || S_q <= 0 || BH * ceil_div(S_q, 256) >= kTargetBlocks)
+    if (D != kD || BH <= 0 || S_q <= 0 || BH * ceil_div(S_q, kBM8) >= kTargetBlocks)
         return pl;
     pl.waves = 4;
     const int64_t units = BH * ceil_div(S_q, 128);
@@ -111,7 +140,7 @@ FlashPlan flash_plan(int64_t BH, int S_q, int S_kv, int D, float tile_us)
         return pl;
     const int64_t tiles = ceil_div(ntiles, std::min(want, ntiles));
     const int64_t splits = ceil_div(ntiles, tiles);
-    if (splits < 2 || (tile_us > 0.0f && double(ntiles - tiles) * tile_us < kSplitCostUs))
+    if (splits < 2)
         return pl;
     pl.splits = int(splits);
     pl.tiles = int(tiles);
@@ -120,21 +149,109 @@ FlashPlan flash_plan(int64_t BH, int S_q, int S_kv, int D, float tile_us)
     return pl;
 }
 
-FlashSplitArgs flash_split_args(const FlashPlan &pl, int64_t BH, int S_q, void *part,
-                                size_t part_bytes)
+// The balanced shape; u == 0 where the query tiles come out even, or where a
+// share would be a whole tile anyway.
+FlashPlan balanced_plan(int64_t BH, int S_q, int S_kv, int D)
+{
+    FlashPlan pl;
+    if (D != kD || BH <= 0 || S_q <= 0 || S_kv <= 0)
+        return pl;
+    const int64_t T = BH * ceil_div(S_q, kBM8), nk = ceil_div(S_kv, kBN);
+    const int64_t tail = T % kTargetBlocks;
+    if (tail == 0 || T > INT32_MAX / 2 || nk > INT32_MAX / kTargetBlocks)
+        return pl;
+    const int64_t u = ceil_div(tail * nk, kTargetBlocks);
+    if (u >= nk)
+        return pl;
+    pl.full = int(T - tail);
+    pl.ntail = int(tail);
+    pl.nk = int(nk);
+    pl.u = int(u);
+    pl.bytes = size_t(tail + ceil_div(tail * nk, u) - 1) * kSlotBytes;
+    return pl;
+}
+
+}  // namespace
+
+FlashPlan flash_plan(int64_t BH, int S_q, int S_kv, int D, const FlashTimes &t, bool causal,
+                     size_t part_bytes, size_t balance_bytes)
+{
+    FlashPlan best;
+    if (D != kD || BH <= 0 || S_q <= 0)
+        return best;
+    const int64_t T = BH * ceil_div(S_q, kBM8), T4 = BH * ceil_div(S_q, 128);
+    const double n = double(ceil_div(S_kv, kBN));
+    const auto rounds = [](int64_t blocks) { return double(ceil_div(blocks, kTargetBlocks)); };
+    // Whole rounds of 8-wave workgroups, and one that fills part of the CUs.
+    const double tail = double(T % kTargetBlocks) / kTargetBlocks;
+    double us = (double(T / kTargetBlocks) + (tail > 0 ? std::max(tail, double(t.part)) : 0)) * n *
+                t.w8;
+    const auto consider = [&](const FlashPlan &pl, double cost) {
+        if (cost < us) {
+            us = cost;
+            best = pl;
+        }
+    };
+    if (T < kTargetBlocks) {
+        FlashPlan small;
+        small.waves = 4;
+        consider(small, rounds(T4) * n * t.w4);
+        const FlashPlan sp = split_plan(BH, S_q, S_kv, D);
+        if (sp.splits > 1 && sp.bytes <= part_bytes)
+            consider(sp, rounds(T4 * sp.splits) * sp.tiles * t.w4 + kSplitCostUs);
+    }
+    const FlashPlan bal = balanced_plan(BH, S_q, S_kv, D);
+    if (bal.u > 0 && !causal && bal.bytes <= balance_bytes)
+        consider(bal, (bal.full / kTargetBlocks * n + bal.u) * t.w8 + kBalanceCostUs);
+    return best;
+}
+
+size_t flash_split_bytes(int64_t BH, int S_q, int S_kv, int D)
+{
+    return split_plan(BH, S_q, S_kv, D).bytes;
+}
+
+size_t flash_balance_bytes(int64_t BH, int S_q, int S_kv, int D, const FlashTimes &t)
+{
+    const FlashPlan pl = flash_plan(BH, S_q, S_kv, D, t, false, SIZE_MAX, SIZE_MAX);
+    return pl.u > 0 ? pl.bytes : 0;
+}
+
+bool flash_fills_gpu(int64_t BH, int S_q, int D)
+{
+    return D != kD || BH <= 0 || S_q <= 0 || BH * ceil_div(S_q, kBM8) >= kTargetBlocks;
+}
+
+FlashSplitArgs flash_split_args(const FlashPlan &pl, int64_t BH, int S_q, const FlashScratch &s,
+                                FlashDeal &deal)
 {
     FlashSplitArgs sa;
-    if (pl.splits < 2 || !part || part_bytes < pl.bytes ||
-        (reinterpret_cast<uintptr_t>(part) & 15u) != 0)
-        return sa;
-    const size_t rows = size_t(pl.splits) * size_t(BH) * size_t(S_q);
-    sa.n = pl.splits;
-    sa.tiles = pl.tiles;
     sa.BH = BH;
-    sa.part = static_cast<float *>(part);
-    sa.ml = reinterpret_cast<float2 *>(static_cast<char *>(part) +
+    size_t rows = 0;
+    if (pl.u > 0) {
+        sa.full = pl.full;
+        sa.ntail = pl.ntail;
+        sa.nk = pl.nk;
+        sa.u = pl.u;
+        deal_pieces(pl.ntail, pl.nk, pl.u, deal, sa.ng, sa.nshorter);
+        sa.part = static_cast<float *>(s.balance);
+        rows = pl.bytes / kSlotBytes * kBM8;
+    } else if (pl.splits > 1) {
+        sa.n = pl.splits;
+        sa.tiles = pl.tiles;
+        sa.part = static_cast<float *>(s.part);
+        rows = size_t(pl.splits) * size_t(BH) * size_t(S_q);
+    }
+    sa.ml = reinterpret_cast<float2 *>(reinterpret_cast<char *>(sa.part) +
                                        round_up256(rows * kD * sizeof(float)));
     return sa;
+}
+
+int64_t flash_blocks(const FlashSplitArgs &sa, int64_t BH, int S_q, int BM)
+{
+    if (sa.u > 0)
+        return sa.full + sa.ng + sa.nshorter;
+    return BH * ceil_div(S_q, BM) * sa.n;
 }
 
 bool launch_flash_combine(const FlashProblem &p, const FlashSplitArgs &sa, hipStream_t st)
@@ -146,13 +263,18 @@ bool launch_flash_combine(const FlashProblem &p, const FlashSplitArgs &sa, hipSt
     a.os = p.os.s;
     a.H = p.H;
     a.S_q = p.S_q;
+    a.n_qtiles = int(ceil_div(p.S_q, kBM8));
     a.sa = sa;
     a.ot = p.ot;
-    a.total = sa.BH * p.S_q * (kD / 4);
+    const bool bal = sa.u > 0;
+    a.total = (bal ? int64_t(sa.ntail) * kBM8 : sa.BH * p.S_q) * (kD / 4);
     const int64_t nblk = ceil_div(a.total, 256);
     if (nblk > INT32_MAX)
         return fail("flash_combine: problem too large for one launch");
-    hipLaunchKernelGGL(flash_combine_kernel, dim3(unsigned(nblk)), dim3(256), 0, st, a);
+    if (bal)
+        hipLaunchKernelGGL(flash_combine_kernel<true>, dim3(unsigned(nblk)), dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL(flash_combine_kernel<false>, dim3(unsigned(nblk)), dim3(256), 0, st, a);
     return hip_ok(hipGetLastError(), "flash_combine_kernel launch");
 }
 

@@ -239,16 +239,59 @@ __device__ __forceinline__ void store_o_rows(float *lds, const f32x16 &o0, const
 // up streaming every (batch, head)'s K/V from HBM.  Renumbered so that the
 // workgroups of one XCD take one contiguous range of ids, the query tiles of
 // a (batch, head), which read the same K/V tiles at about the same time, run
-// on one XCD and share its L2.  A bijection on [0, gridDim.x) for every grid
+// on one XCD and share its L2.  A bijection on [0, n) for every grid
 // size (the first n % 8 XCDs take one id more), so only locality depends on
 // the dispatch order, never the result.
-constexpr unsigned kXcds = 8;
-__device__ __forceinline__ int xcd_major_block()
+// `i` of `n` workgroups whose first one went to XCD 0.
+__device__ __forceinline__ int xcd_major(unsigned i, unsigned n)
 {
-    const unsigned n = gridDim.x, i = blockIdx.x, x = i % kXcds;
-    const unsigned q = n / kXcds, r = n % kXcds;
+    const unsigned x = i % kXcds, q = n / kXcds, r = n % kXcds;
     return int(x * q + (x < r ? x : r) + i / kXcds);
 }
+
+__device__ __forceinline__ int xcd_major_block() { return xcd_major(blockIdx.x, gridDim.x); }
+
+// The part of an attention that this workgroup computes (FlashPlan): one query
+// tile, whole or one split of its keys, or part of one of a balanced grid's
+// tail tiles.  Uniform over the workgroup.
+struct FlashWork {
+    int qt, bh;    // query tile and batch * H + head
+    int j0, jn;    // first key tile and the most of them (0: nothing to do)
+    int64_t prow;  // partial row of the query tile's first row; -1: O itself
+
+    __device__ __forceinline__ FlashWork(const FlashSplitArgs &sa, const FlashWhole &,
+                                         int n_qtiles, int S_q, int BM)
+    {
+        const int blk = xcd_major(blockIdx.x, gridDim.x);
+        const int sp = blk % sa.n;
+        qt = (blk / sa.n) % n_qtiles;
+        bh = (blk / sa.n) / n_qtiles;
+        j0 = sp * sa.tiles;
+        jn = sa.tiles;
+        prow = sa.n > 1 ? (int64_t(sp) * sa.BH + bh) * S_q + int64_t(qt) * BM : -1;
+    }
+    __device__ __forceinline__ FlashWork(const FlashSplitArgs &sa, const FlashDeal &deal,
+                                         int n_qtiles, int, int BM)
+    {
+        if (int(blockIdx.x) < sa.full) {
+            const int blk = xcd_major(blockIdx.x, sa.full);
+            qt = blk % n_qtiles;
+            bh = blk / n_qtiles;
+            j0 = 0;
+            jn = sa.nk;
+            prow = -1;
+            return;
+        }
+        // sa.full is a multiple of 256, so the pieces start at XCD 0.
+        const FlashPiece p = flash_piece(int(blockIdx.x) - sa.full, sa.ntail, sa.nk, sa.u, sa.ng,
+                                         deal);
+        j0 = p.j0;
+        jn = p.jn;
+        qt = (sa.full + p.t) % n_qtiles;
+        bh = (sa.full + p.t) / n_qtiles;
+        prow = int64_t(p.t + p.g) * BM;
+    }
+};
 
 inline bool aligned(const void *ptr, unsigned m)
 {

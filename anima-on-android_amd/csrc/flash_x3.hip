@@ -52,16 +52,16 @@ struct X3Args {
     float c;  // scale * log2(e), > 0
     int causal;
     int dma32;  // K/V^T tile rows fit 32-bit byte offsets from the tile start
-    FlashSplitArgs split;  // n == 1: write O; n > 1: write this split's partial
-    TermOut ot;            // n == 1 and ot.t set: O as bf16 terms
+    FlashSplitArgs split;  // which parts this workgroup computes
+    TermOut ot;            // whole tiles, ot.t set: O as bf16 terms
     // Raw query rows (RawQ) in place of q's term rows when qx is set.
     const float *qx, *qw, *qf;
     int64_t rqb, rqh, rqs;
     float eps;
 };
 
-template <int NW>
-__global__ __launch_bounds__(NW * 64, 1) void flash_x3_d128(X3Args a)
+template <int NW, typename Deal>
+__global__ __launch_bounds__(NW * 64, 1) void flash_x3_d128(X3Args a, Deal deal)
 {
     constexpr int NT = NW * 64;
     constexpr int BM = NW * 32;
@@ -80,13 +80,13 @@ __global__ __launch_bounds__(NW * 64, 1) void flash_x3_d128(X3Args a)
     const int col = lane & 31;
     const int half = lane >> 5;
 
-    const int blk = xcd_major_block();
-    const int sp = blk % a.split.n;
-    const int qt = (blk / a.split.n) % a.n_qtiles;
-    const int bh = (blk / a.split.n) / a.n_qtiles;
+    const FlashWork work(a.split, deal, a.n_qtiles, a.S_q, BM);
+    if (work.jn == 0)
+        return;
+    const int bh = work.bh;
     const int b = bh / a.H;
     const int h = bh - b * a.H;
-    const int q_tile0 = qt * BM;
+    const int q_tile0 = work.qt * BM;
     const int qrow = q_tile0 + wave * 32 + col;
 
     const u16 *qp = a.q + b * a.qb + h * a.qh;
@@ -96,9 +96,9 @@ __global__ __launch_bounds__(NW * 64, 1) void flash_x3_d128(X3Args a)
     int kv_end = a.S_kv;
     if (a.causal)
         kv_end = min(kv_end, min(a.S_q, q_tile0 + BM));
-    // Key tiles [j0, j0 + ntiles) of this split (all of them when unsplit).
-    const int j0 = sp * a.split.tiles;
-    const int ntiles = max(0, min((kv_end + kBN - 1) / kBN - j0, a.split.tiles));
+    // Key tiles [j0, j0 + ntiles) of this part (all of them when unsplit).
+    const int j0 = work.j0;
+    const int ntiles = max(0, min((kv_end + kBN - 1) / kBN - j0, work.jn));
 
     // LDS layouts, unpadded, XOR-swizzled (16-byte chunks):
     //   K   [64 keys][256]: chunk c (0..31; hi 0..15, lo 16..31) of key row r
@@ -371,9 +371,9 @@ __global__ __launch_bounds__(NW * 64, 1) void flash_x3_d128(X3Args a)
     float *op = a.o + b * a.ob + h * a.oh + row0 * a.os;
     int64_t ostride = a.os;
     u16 *tp = a.ot.t ? a.ot.t + b * a.ot.tb + h * a.ot.th + row0 * a.ot.ts : nullptr;
-    if (a.split.n > 1) {
+    if (work.prow >= 0) {
         tp = nullptr;
-        const int64_t prow0 = (int64_t(sp) * a.split.BH + bh) * a.S_q + row0;
+        const int64_t prow0 = work.prow + wave * 32;
         op = a.split.part + prow0 * kD;
         ostride = kD;
         if (half == 0 && qrow < a.S_q)
@@ -441,22 +441,22 @@ __global__ __launch_bounds__(256) void vt_pack_terms_kernel(PackArgs a)
     }
 }
 
-template <int NW>
-bool launch_d128(const X3Args &a, int64_t BH, hipStream_t st)
+template <int NW, typename Deal>
+bool launch_d128(const X3Args &a, const Deal &deal, int64_t BH, hipStream_t st)
 {
     constexpr int BM = NW * 32;
     X3Args g = a;
     g.n_qtiles = (g.S_q + BM - 1) / BM;
-    const int64_t nblk = BH * g.n_qtiles * g.split.n;
+    const int64_t nblk = flash_blocks(g.split, BH, g.S_q, BM);
     if (nblk > INT32_MAX)
         return fail("flash_x3: problem too large for one launch");
-    hipLaunchKernelGGL(flash_x3_d128<NW>, dim3(unsigned(nblk)), dim3(NW * 64), 0, st, g);
+    hipLaunchKernelGGL((flash_x3_d128<NW, Deal>), dim3(unsigned(nblk)), dim3(NW * 64), 0, st, g, deal);
     return hip_ok(hipGetLastError(), "flash_x3_d128 launch");
 }
 
 }  // namespace
 
-bool launch_flash_x3(const FlashProblem &p, hipStream_t st, void *part, size_t part_bytes)
+bool launch_flash_x3(const FlashProblem &p, hipStream_t st, const FlashScratch &scr)
 {
     const int64_t BH = int64_t(p.B) * p.H;
     if (BH == 0 || p.S_q == 0)
@@ -520,11 +520,15 @@ bool launch_flash_x3(const FlashProblem &p, hipStream_t st, void *part, size_t p
     a.qf = p.rq.freqs;
     a.rqb = p.rq.s.b; a.rqh = p.rq.s.h; a.rqs = p.rq.s.s;
     a.eps = p.rq.eps;
-    const FlashPlan pl = flash_plan(BH, p.S_q, p.S_kv, p.D, kTileUsX3);
-    a.split = flash_split_args(pl, BH, p.S_q, part, part_bytes);
-    if (!(pl.waves == 4 ? launch_d128<4>(a, BH, st) : launch_d128<8>(a, BH, st)))
+    const FlashPlan pl = flash_plan(BH, p.S_q, p.S_kv, p.D, kTimesX3, p.causal, scr.part_bytes,
+                                    scr.balance_bytes);
+    FlashDeal deal;
+    a.split = flash_split_args(pl, BH, p.S_q, scr, deal);
+    if (!(pl.waves == 4 ? launch_d128<4>(a, FlashWhole{}, BH, st)
+          : pl.u > 0    ? launch_d128<8>(a, deal, BH, st)
+                        : launch_d128<8>(a, FlashWhole{}, BH, st)))
         return false;
-    return a.split.n == 1 || launch_flash_combine(p, a.split, st);
+    return (a.split.n == 1 && a.split.u == 0) || launch_flash_combine(p, a.split, st);
 }
 
 bool launch_vt_pack_terms(const float *v, Strides vs, uint16_t *vt, Strides vts, int B, int H,

@@ -20,11 +20,16 @@
 #include <mutex>
 #include <string>
 
-static __device__ __align__(256) unsigned char scratch[ANIMA_HIP_STATIC_SCRATCH_BYTES];
+// The scratch every call needs, and behind it room for the partials of a
+// balanced flash grid, so that every accepted problem runs the kernels
+// anima_hip_attention_dev runs.
+static __device__ __align__(256) unsigned char
+    scratch[ANIMA_HIP_STATIC_SCRATCH_BYTES + anima_hip::kMaxFlashBalanceBytes];
 
 namespace {
 
 constexpr size_t kStaticScratchBytes = size_t(ANIMA_HIP_STATIC_SCRATCH_BYTES);
+static_assert(kStaticScratchBytes % 256 == 0, "the partials follow 16-byte aligned");
 constexpr int kMaxDevices = 64;
 
 std::mutex g_mu;
@@ -101,6 +106,8 @@ bool anima_hip_attention_static_dev(const float *q, const float *k, const float 
     in.D = D;
     in.eps = eps;
     in.mode = am;
+    in.balance = static_cast<char *>(ws) + kStaticScratchBytes;
+    in.balance_bytes = kMaxFlashBalanceBytes;
     return run_attention(in, ws, static_cast<hipStream_t>(stream));
 }
 

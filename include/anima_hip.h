@@ -313,7 +313,11 @@ bool anima_hip_linear_dev(const float *a, int64_t lda, const uint16_t *w, int64_
                           int64_t ldc, int M, int N, int K, int mode, void *scratch,
                           size_t scratch_bytes, void *stream);
 
-/* Device scratch needed by anima_hip_attention_dev for these sizes (bytes). */
+/* Device scratch for anima_hip_attention_dev at these sizes (bytes).  Where
+ * the query tiles of 256 rows do not come out even over the GPU's 256 CUs,
+ * up to 65 MiB of it hold partial results of a grid that shares their keys
+ * out; a call with that much less runs too, on whole query tiles (results
+ * differ by summation order).  The other size queries are alike. */
 size_t anima_hip_attention_scratch_bytes(int B, int S_q, int Bk, int S_kv, int H, int D,
                                          int mode);
 
@@ -350,10 +354,10 @@ bool anima_hip_attention_terms_dev(const float *q, const float *k, const float *
  * device memory (code under HIP graph capture, serving loops that forbid
  * hipMalloc).  Same arguments, kernels and results as
  * anima_hip_attention_dev; the scratch is a static device array of
- * ANIMA_HIP_STATIC_SCRATCH_BYTES that each GPU holds from the first call
- * made on it until the process ends (measured on MI355X: the library's
- * other entries leave it unreserved; free device memory drops by 194 MiB
- * at the first static call).  The array's device address is looked up once
+ * ANIMA_HIP_STATIC_SCRATCH_BYTES, and 65 MiB for the partial results of
+ * balanced grids, that each GPU holds from the first call made on it until
+ * the process ends (the library's other entries leave it unreserved; free
+ * device memory drops by about 260 MiB at the first static call).  The array's device address is looked up once
  * per GPU, at that first call, and kept: resetting a device
  * (hipDeviceReset) while the library is loaded is not supported.  The first
  * call may itself be captured into a HIP graph.  A problem whose
