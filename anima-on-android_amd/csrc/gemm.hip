@@ -7,17 +7,22 @@
 // projections k_proj / v_proj (anima_rt/scripts/numpy_dit.py:277-281), whose
 // results the context K/V cache keeps for every denoise step.
 //
-// Block tile 128x128, K chunk 32, 4 waves in a 2x2 grid each owning 64x64
-// (four 32x32 MFMA accumulators).  Operands are staged through LDS as f32
-// (bf16 weights widened on the way in); every global access is bounds-checked
-// so any M, N, K and any leading dimensions are accepted.
-#include "common.h"
+// Two kernels:
+//   gemm_tile_kernel  f32 weights, 16-byte aligned rows, K a multiple of 32: the
+//                     operands reach LDS by DMA;
+//   gemm_kernel       everything else: block tile 128x128, K chunk 32, 4 waves
+//                     in a 2x2 grid each owning 64x64 (four 32x32 MFMA
+//                     accumulators), operands staged through LDS as f32 element
+//                     by element (bf16 weights widened on the way in); every
+//                     global access is bounds-checked so any M, N, K and any
+//                     leading dimensions are accepted.
+#include "flash_tile.h"
 
 namespace anima_hip {
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+using flash_tile::f32x16;
+using flash_tile::f32x4;
 
 constexpr int kBM = 128, kBN = 128, kBK = 32;
 constexpr int kPitch = kBK + 4;  // floats per LDS row
@@ -99,6 +104,106 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g)
             }
 }
 
+// C = A . W^T on f32 MFMA from DMA-staged tiles: 64 x 64 of C per workgroup, 4
+// waves in a 2x2 grid each owning 32 x 32.  Bound by the f32 MFMA pipe, which
+// takes 64 cycles per 32x32x2 product: a chunk of 32 k needs 16 bytes per clock
+// from L2 and 32 from LDS, inside what a CU gets (35 and 128), so the small tile
+// costs little and comes out more even over the CUs.  Two stages of one chunk
+// (32 KiB, five workgroups to a CU), one barrier per chunk; other workgroups'
+// products fill a wave's waits.  Two accumulators take the products of even and
+// odd k: shorter chains, and rounding errors 0.7 times one chain's.
+// Whole calls on MI355X, before (gemm_kernel) and now: 2400x2048x2048 785 ->
+// 187 us (108 TFLOP/s), 8192x2048x2048 1061 -> 537 (128), 512x2048x8192 2575 ->
+// 155, 100x2048x2048 365 -> 40.  Measured beside it at the first two shapes:
+// 128 x 128 tiles, two workgroups to a CU 257 / 518 us; three stages and three
+// workgroups 191 / 567; one accumulator 188 / 542; no raised priority 191 / 558.
+//
+// A chunk's row holds 32 k as eight 16-byte pieces; piece c of row r is at
+// c ^ ((r >> 1) & 7), so the 16 rows that a fragment read serves per clock fall
+// into 16 different bank groups.  Lane half h contracts k = 16h + t (t = 0..15)
+// of the chunk, for A and W alike.
+struct TileArgs {
+    const float *a, *w;
+    float *c;
+    int64_t lda, ldw, ldc;
+    int M, N, chunks, n_tiles_n;
+};
+
+constexpr int kT = 64;
+
+__global__ __launch_bounds__(256, 5) void gemm_tile_kernel(TileArgs g)
+{
+    constexpr int kRows = 2 * kT;             // A rows, then W rows
+    constexpr int kCopies = kRows * 8 / 256;  // 16-byte copies per thread and chunk
+    __shared__ __attribute__((aligned(16))) float ring[2][kRows * kBK];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 31, half = lane >> 5;
+    const int blk = flash_tile::xcd_major_block();
+    const int m0 = blk / g.n_tiles_n * kT, n0 = blk % g.n_tiles_n * kT;
+
+    // Copy i of this wave fills pieces (wave*kCopies + i)*64 + lane of the
+    // stage; rows past M or N copy the last row (their C is not stored).
+    const float *src[kCopies];
+#pragma unroll
+    for (int i = 0; i < kCopies; ++i) {
+        const int f = (wave * kCopies + i) * 64 + lane, r = f >> 3;
+        const int c = (f & 7) ^ ((r >> 1) & 7);
+        src[i] = (r < kT ? g.a + int64_t(min(m0 + r, g.M - 1)) * g.lda
+                         : g.w + int64_t(min(n0 + r - kT, g.N - 1)) * g.ldw) +
+                 4 * c;
+    }
+    auto copy = [&](int chunk) {
+#pragma unroll
+        for (int i = 0; i < kCopies; ++i)
+            flash_tile::dma16(reinterpret_cast<const flash_tile::u16 *>(src[i] + chunk * kBK),
+                              reinterpret_cast<flash_tile::u16 *>(
+                                  &ring[chunk & 1][(wave * kCopies + i) * 256]));
+    };
+    copy(0);
+
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    const int sw = (col >> 1) & 7;
+    f32x16 acc0 = {}, acc1 = {};
+    for (int k = 0; k < g.chunks; ++k) {
+        flash_tile::wait_vmcnt<0>();
+        flash_tile::ring_barrier();
+        // The other stage was read in the previous iteration.
+        if (k + 1 < g.chunks)
+            copy(k + 1);
+        const float *ar = ring[k & 1] + (wm + col) * kBK;
+        const float *wr = ring[k & 1] + (kT + wn + col) * kBK;
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int t4 = 0; t4 < 4; ++t4) {
+            const int piece = 4 * ((4 * half + t4) ^ sw);
+            const f32x4 av = *reinterpret_cast<const f32x4 *>(ar + piece);
+            const f32x4 wv = *reinterpret_cast<const f32x4 *>(wr + piece);
+            acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(av.x, wv.x, acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(av.y, wv.y, acc1, 0, 0, 0);
+            acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(av.z, wv.z, acc0, 0, 0, 0);
+            acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(av.w, wv.w, acc1, 0, 0, 0);
+        }
+        __builtin_amdgcn_s_setprio(0);
+    }
+    acc0 += acc1;
+    // Register r, lane l: row acc_row(r, half), column l%32.
+    const int gn = n0 + wn + col;
+    float *c = g.c + int64_t(m0 + wm) * g.ldc + gn;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const int row = flash_tile::acc_row(r, half);
+        if (m0 + wm + row < g.M && gn < g.N)
+            c[row * g.ldc] = acc0[r];
+    }
+}
+
+bool tile_supported(const float *a, int64_t lda, const void *w, bool w_bf16, int64_t ldw, int K)
+{
+    return !w_bf16 && K > 0 && K % kBK == 0 && lda % 4 == 0 && ldw % 4 == 0 &&
+           flash_tile::aligned(a, 16) && flash_tile::aligned(w, 16);
+}
+
 }  // namespace
 
 bool launch_gemm(const float *a, int64_t lda, const void *w, bool w_bf16, int64_t ldw, float *c,
@@ -108,6 +213,16 @@ bool launch_gemm(const float *a, int64_t lda, const void *w, bool w_bf16, int64_
         return fail("gemm: negative dimension");
     if (M == 0 || N == 0)
         return true;  // K == 0 runs the kernel, which then stores zeros
+    if (tile_supported(a, lda, w, w_bf16, ldw, K)) {
+        const int64_t n_tiles_n = (int64_t(N) + kT - 1) / kT;
+        const int64_t nblk = (int64_t(M) + kT - 1) / kT * n_tiles_n;
+        if (nblk > INT32_MAX)
+            return fail("gemm: problem too large for one launch");
+        const TileArgs t{a, static_cast<const float *>(w), c, lda, ldw, ldc, M, N, K / kBK,
+                         int(n_tiles_n)};
+        hipLaunchKernelGGL(gemm_tile_kernel, dim3(unsigned(nblk)), dim3(256), 0, st, t);
+        return hip_ok(hipGetLastError(), "gemm_tile_kernel launch");
+    }
     GemmArgs g;
     g.a = a;
     g.w = w;
