@@ -1482,7 +1482,9 @@ bool anima_hip_qkv_projection_dev(const float *x, int64_t ldx, const uint16_t *w
     p.H = H;
     p.eps = eps;
     p.mode = mode == ANIMA_HIP_F32 ? kAttnF32 : kAttnF32X3;
-    return launch_gemm_f32a_qkv(x, ldx, w_qkv, ldw, K, p, pick_stream(stream));
+    const int64_t part = int64_t(H) * 128 * ldw;
+    const uint16_t *const w[3] = {w_qkv, w_qkv + part, w_qkv + 2 * part};
+    return launch_gemm_f32a_qkv(x, ldx, w, ldw, K, p, pick_stream(stream));
 }
 
 bool anima_hip_gemm_dev(const float *a, int64_t lda, const void *w, int w_bf16, int64_t ldw,

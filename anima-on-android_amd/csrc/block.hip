@@ -369,26 +369,67 @@ bool run_attention_block(const BlockProblem &p, void *scratch, size_t scratch_by
     void *attn = take(s.attn);
     void *lin = take(s.lin);
 
-    // x_m as bf16 terms, then the projections of NumpyAttention.forward
+    // x_m, then the projections of NumpyAttention.forward
     // (numpy_dit.py:273-281): q from x_m, and k/v from x_m (self) or the
-    // cached context projections (cross).
-    if (!launch_ln_modulate(p.x, Dm, p.mod, 3 * int64_t(Dm), hi, lo, M, S, Dm, p.eps, st))
-        return false;
-    if (!launch_linear_terms(hi, lo, p.wq, Dm, q, HD, int(M), HD, Dm, st))
-        return false;
-    if (!cross && (!launch_linear_terms(hi, lo, p.wk, Dm, k, HD, int(M), HD, Dm, st) ||
-                   !launch_linear_terms(hi, lo, p.wv, Dm, v, HD, int(M), HD, Dm, st)))
-        return false;
-
+    // cached context projections (cross).  In the f32 modes self-attention's
+    // three products run as one grid on f32 rows of x_m where 256 x 256 tiles
+    // of all three fill the GPU (2304 tokens, B = 2, Dm = 2048: three grids of
+    // the two-plane kernel took 288 us in six rounds of tiles that fill 1.1
+    // each), which can write the attention's prepared operands in place of q,
+    // k and v (H even, S a multiple of 64; the prologue pass, 48 us there, goes
+    // away).  Otherwise bf16 terms of x_m and a product each.
     AttnInputs in;
+    const uint16_t *const w3[3] = {p.wq, p.wk, p.wv};
+    const float *xm = reinterpret_cast<const float *>(hi);
+    QkvPrep qp;
+    bool prep = false, three = false;
+    if (!cross && !bf16) {
+        qp.qo = q;
+        qp.ko = k;
+        qp.vo = v;
+        qp.w[0] = p.q_norm_w;
+        qp.w[1] = p.k_norm_w;
+        qp.freqs = p.freqs;
+        qp.B = B;
+        qp.S = S;
+        qp.H = H;
+        qp.eps = p.eps;
+        qp.mode = p.mode;
+        prep = D == 128 && gemm_f32a_qkv_supported(xm, Dm, w3, Dm, Dm, qp);
+        three = prep || (M <= INT32_MAX &&
+                         gemm_f32a_three_supported(int(M), HD, Dm, Dm, Dm, HD, xm, w3, q));
+    }
+    if (!launch_ln_modulate(p.x, Dm, p.mod, 3 * int64_t(Dm), three ? nullptr : hi,
+                            three ? nullptr : lo, M, S, Dm, p.eps, st, nullptr, nullptr, nullptr, 0,
+                            0, 1, three ? reinterpret_cast<float *>(hi) : nullptr))
+        return false;
+    if (prep) {
+        if (!launch_gemm_f32a_qkv(xm, Dm, w3, Dm, Dm, qp, st))
+            return false;
+        in.q_prep = qp.qo;
+        in.k_prep = qp.ko;
+        in.v_prep = qp.vo;
+    } else if (three) {
+        if (!launch_gemm_f32a_three(xm, Dm, w3, Dm, q, k - q, HD, int(M), HD, Dm, st))
+            return false;
+    } else {
+        if (!launch_linear_terms(hi, lo, p.wq, Dm, q, HD, int(M), HD, Dm, st))
+            return false;
+        if (!cross && (!launch_linear_terms(hi, lo, p.wk, Dm, k, HD, int(M), HD, Dm, st) ||
+                       !launch_linear_terms(hi, lo, p.wv, Dm, v, HD, int(M), HD, Dm, st)))
+            return false;
+    }
+
     in.q = q;
     in.q_norm_w = p.q_norm_w;
     in.freqs = cross ? nullptr : p.freqs;
     in.k = k;
     in.v = v;
     in.k_norm_w = p.k_norm_w;
-    in.k_prep = p.k_prep;
-    in.v_prep = p.v_prep;
+    if (cross) {
+        in.k_prep = p.k_prep;
+        in.v_prep = p.v_prep;
+    }
     in.out = o;
     in.B = B;
     in.Bk = cross ? p.Bk : B;

@@ -240,6 +240,14 @@ bool gemm_f32a_supported(int M, int N, int K, int64_t lda, int64_t ldw, int64_t 
                          const float *a, const void *w, const void *c);
 bool launch_gemm_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, float *c,
                       int64_t ldc, int M, int N, int K, bool two_terms, hipStream_t st);
+// Three two-term products of the same a in one grid: a . w[i]^T [M][N] to
+// c + i * c_step, each bit-identical to launch_gemm_f32a's; N a multiple of
+// 256, and a grid of at least 256 tiles over all three.
+bool gemm_f32a_three_supported(int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
+                               const float *a, const uint16_t *const w[3], const float *c);
+bool launch_gemm_f32a_three(const float *a, int64_t lda, const uint16_t *const w[3], int64_t ldw,
+                            float *c, int64_t c_step, int64_t ldc, int M, int N, int K,
+                            hipStream_t st);
 
 // Small-M bf16 GEMM (gemm_bf16.hip): C[M,N] = a0 . W^T (+ a1 . W^T) with bf16
 // activation terms a0 (a1 null for one term) [M][lda], bf16 W [N][ldw], f32
@@ -390,9 +398,9 @@ struct PrepProblem {
 bool prep_qkv_supported(const PrepProblem &p);  // D == 128, 16-byte alignment
 bool launch_prep_qkv(const PrepProblem &p, hipStream_t st);
 // A self-attention's fused q/k/v projection with that one-launch prologue as
-// its epilogue (gemm_f32a.hip): a [B*S][lda] f32 activations times the
-// stacked bf16 weights w [3*H*128][ldw] (q rows, then k, then v), in the f32
-// modes' exact two-term product.  Instead of the product's f32 columns the
+// its epilogue (gemm_f32a.hip): a [B*S][lda] f32 activations times the bf16
+// weights of q, k and v, w[i] [H*128][ldw] (stacked in one buffer or not), in
+// the f32 modes' exact two-term product.  Instead of the product's f32 columns the
 // kernel writes the attention operands: qo / ko as launch_prep_qkv writes
 // them (RMSNorm with w[0] / w[1], RoPE with freqs), and vo as the x3
 // kernel's term V^T (kAttnF32X3) or dense f32 V rows [B, S, H, 128]
@@ -408,10 +416,10 @@ struct QkvPrep {
     float eps = 1e-6f;
     AttnMode mode = kAttnF32X3;
 };
-bool gemm_f32a_qkv_supported(const float *a, int64_t lda, const void *w, int64_t ldw, int K,
-                             const QkvPrep &p);
-bool launch_gemm_f32a_qkv(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, int K,
-                          const QkvPrep &p, hipStream_t st);
+bool gemm_f32a_qkv_supported(const float *a, int64_t lda, const uint16_t *const w[3], int64_t ldw,
+                             int K, const QkvPrep &p);
+bool launch_gemm_f32a_qkv(const float *a, int64_t lda, const uint16_t *const w[3], int64_t ldw,
+                          int K, const QkvPrep &p, hipStream_t st);
 size_t prepared_k_bytes(int Bk, int S_kv, int H, int D, AttnMode mode);
 size_t prepared_v_bytes(int Bk, int S_kv, int H, int D, AttnMode mode);
 // Scratch run_attention needs, and what it can use beside that

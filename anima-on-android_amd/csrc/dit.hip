@@ -690,9 +690,10 @@ bool dit_sublayer(const anima_hip_dit *d, const BlockWeights &bw, int kind, floa
         qp.H = c.heads;
         qp.mode = d->attn;
     }
+    const uint16_t *const w3[3] = {bw.w_qkv, bw.w_qkv + HD * d->ld_d, bw.w_qkv + 2 * HD * d->ld_d};
     const bool fused_qkv = try_fused &&
-                           gemm_f32a_qkv_supported(reinterpret_cast<const float *>(terms), D,
-                                                   bw.w_qkv, d->ld_d, D, qp);
+                           gemm_f32a_qkv_supported(reinterpret_cast<const float *>(terms), D, w3,
+                                                   d->ld_d, D, qp);
     if (fused_qkv) {
         if (!launch_ln_modulate(x, D, mod, 3 * int64_t(D), nullptr, nullptr, M, int(S), D, 1e-6f,
                                 st, x, pend_y, pend_y ? pend_mod + 2 * int64_t(D) : nullptr,
@@ -741,8 +742,8 @@ bool dit_sublayer(const anima_hip_dit *d, const BlockWeights &bw, int kind, floa
     in.balance = balance;
     in.balance_bytes = balance_bytes;
     if (fused_qkv) {
-        if (!launch_gemm_f32a_qkv(reinterpret_cast<const float *>(terms), D, bw.w_qkv, d->ld_d, D,
-                                  qp, st))
+        if (!launch_gemm_f32a_qkv(reinterpret_cast<const float *>(terms), D, w3, d->ld_d, D, qp,
+                                  st))
             return false;
         in.q_prep = qp.qo;
         in.k_prep = qp.ko;

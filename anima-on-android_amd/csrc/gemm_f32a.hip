@@ -84,10 +84,12 @@ struct FaQkv {
 
 struct FaArgs {
     const float *a;   // [M][lda]
-    const u16 *w;     // [N][ldw]
+    // The N columns in parts of part_n (a multiple of 256, or N itself): part
+    // i has weights w[i] [part_n][ldw] and its C at c + i * c_step.
+    const u16 *w[3];
     float *c;         // [M][ldc]
-    int64_t lda, ldw, ldc;
-    int M, N, tiles_n, chunks;
+    int64_t lda, ldw, ldc, c_step;
+    int M, N, part_n, tiles_n, chunks;
     FaQkv qkv;        // QKV kernels only
 };
 
@@ -306,7 +308,9 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
         woff[i] = unsigned(int64_t(rr) * g.ldw * 2 + 16 * pc);
     }
     const char *asrc = reinterpret_cast<const char *>(g.a + int64_t(row0) * g.lda);
-    const char *wsrc = reinterpret_cast<const char *>(g.w + int64_t(col0) * g.ldw);
+    const int part = col0 / g.part_n, pcol0 = col0 - part * g.part_n;
+    const u16 *wp = part == 0 ? g.w[0] : part == 1 ? g.w[1] : g.w[2];
+    const char *wsrc = reinterpret_cast<const char *>(wp + int64_t(pcol0) * g.ldw);
     // Copy i (0 .. kCopies - 1) of this wave for chunk c into `stage`: the
     // A windows first, then the W windows.
     auto dma_one = [&](int c, int stage, int i) {
@@ -428,12 +432,13 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
 #pragma unroll
     for (int nb = 0; nb < kFaNB; ++nb) {
         const int n = col0 + 32 * nb + col;
+        float *c = g.c + part * g.c_step + pcol0 + 32 * nb + col;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int m = row0 + wave * 32 + acc_row(r, half);
             if (!full && (m >= g.M || n >= g.N))
                 continue;
-            __builtin_nontemporal_store(acc[nb][r], g.c + int64_t(m) * g.ldc + n);
+            __builtin_nontemporal_store(acc[nb][r], c + int64_t(m) * g.ldc);
         }
     }
 }
@@ -457,21 +462,25 @@ bool gemm_f32a_supported(int M, int N, int K, int64_t lda, int64_t ldw, int64_t 
            int64_t(kFaBN) * ldw * 2 < (int64_t(1) << 31);
 }
 
-bool launch_gemm_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, float *c,
-                      int64_t ldc, int M, int N, int K, bool two_terms, hipStream_t st)
+namespace {
+// One part of N columns, or three of part_n.
+bool launch_parts(const float *a, int64_t lda, const uint16_t *const *w, int parts, int64_t ldw,
+                  float *c, int64_t c_step, int64_t ldc, int M, int part_n, int K, bool two_terms,
+                  hipStream_t st)
 {
-    if (!gemm_f32a_supported(M, N, K, lda, ldw, ldc, a, w, c))
-        return fail("gemm_f32a: unsupported shape or alignment");
-    FaArgs g;
+    FaArgs g{};
     g.a = a;
-    g.w = w;
+    for (int i = 0; i < parts; ++i)
+        g.w[i] = w[i];
     g.c = c;
     g.lda = lda;
     g.ldw = ldw;
     g.ldc = ldc;
+    g.c_step = c_step;
     g.M = M;
-    g.N = N;
-    g.tiles_n = (N + kFaBN - 1) / kFaBN;
+    g.N = parts * part_n;
+    g.part_n = part_n;
+    g.tiles_n = (g.N + kFaBN - 1) / kFaBN;
     g.chunks = K / kFaBK;
     const dim3 grid(unsigned(((M + kFaBM - 1) / kFaBM) * g.tiles_n)), block(kFaWaves * 64);
     if (two_terms)
@@ -480,9 +489,34 @@ bool launch_gemm_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t ld
         hipLaunchKernelGGL((gemm_f32a_kernel<1, false>), grid, block, 0, st, g);
     return hip_ok(hipGetLastError(), "gemm_f32a_kernel launch");
 }
+}  // namespace
 
-bool gemm_f32a_qkv_supported(const float *a, int64_t lda, const void *w, int64_t ldw, int K,
-                             const QkvPrep &p)
+bool launch_gemm_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, float *c,
+                      int64_t ldc, int M, int N, int K, bool two_terms, hipStream_t st)
+{
+    if (!gemm_f32a_supported(M, N, K, lda, ldw, ldc, a, w, c))
+        return fail("gemm_f32a: unsupported shape or alignment");
+    return launch_parts(a, lda, &w, 1, ldw, c, 0, ldc, M, N, K, two_terms, st);
+}
+
+bool gemm_f32a_three_supported(int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
+                               const float *a, const uint16_t *const w[3], const float *c)
+{
+    return N % kFaBN == 0 && N <= INT32_MAX / 3 && aligned(w[1], 16) && aligned(w[2], 16) &&
+           ldc >= N && gemm_f32a_supported(M, 3 * N, K, lda, ldw, 3 * ldc, a, w[0], c);
+}
+
+bool launch_gemm_f32a_three(const float *a, int64_t lda, const uint16_t *const w[3], int64_t ldw,
+                            float *c, int64_t c_step, int64_t ldc, int M, int N, int K,
+                            hipStream_t st)
+{
+    if (!gemm_f32a_three_supported(M, N, K, lda, ldw, ldc, a, w, c))
+        return fail("gemm_f32a: unsupported shape or alignment (three products)");
+    return launch_parts(a, lda, w, 3, ldw, c, c_step, ldc, M, N, K, true, st);
+}
+
+bool gemm_f32a_qkv_supported(const float *a, int64_t lda, const uint16_t *const w[3], int64_t ldw,
+                             int K, const QkvPrep &p)
 {
     const auto al = [](const void *x) { return (reinterpret_cast<uintptr_t>(x) & 15) == 0; };
     if ((p.mode != kAttnF32 && p.mode != kAttnF32X3) || p.B <= 0 || p.S <= 0 || p.H <= 0 ||
@@ -491,13 +525,13 @@ bool gemm_f32a_qkv_supported(const float *a, int64_t lda, const void *w, int64_t
     const int64_t M = int64_t(p.B) * p.S, HD = int64_t(p.H) * 128;
     if (M > INT32_MAX || 3 * HD > INT32_MAX)
         return false;
-    return p.qo && p.ko && p.vo && al(p.qo) && al(p.ko) && al(p.vo) && (!p.w[0] || al(p.w[0])) &&
+    return al(w[1]) && al(w[2]) && p.qo && p.ko && p.vo && al(p.qo) && al(p.ko) && al(p.vo) && (!p.w[0] || al(p.w[0])) &&
            (!p.w[1] || al(p.w[1])) && (!p.freqs || al(p.freqs)) &&
-           gemm_f32a_supported(int(M), int(3 * HD), K, lda, ldw, 3 * HD, a, w, p.qo);
+           gemm_f32a_supported(int(M), int(3 * HD), K, lda, ldw, 3 * HD, a, w[0], p.qo);
 }
 
-bool launch_gemm_f32a_qkv(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, int K,
-                          const QkvPrep &p, hipStream_t st)
+bool launch_gemm_f32a_qkv(const float *a, int64_t lda, const uint16_t *const w[3], int64_t ldw,
+                          int K, const QkvPrep &p, hipStream_t st)
 {
     if (!gemm_f32a_qkv_supported(a, lda, w, ldw, K, p))
         return fail("gemm_f32a_qkv: unsupported mode, shape or alignment (f32 or f32x3 mode, "
@@ -505,11 +539,13 @@ bool launch_gemm_f32a_qkv(const float *a, int64_t lda, const uint16_t *w, int64_
                     "of at least 256 tiles)");
     FaArgs g{};
     g.a = a;
-    g.w = w;
+    for (int i = 0; i < 3; ++i)
+        g.w[i] = w[i];
     g.lda = lda;
     g.ldw = ldw;
     g.M = p.B * p.S;
     g.N = 3 * p.H * 128;
+    g.part_n = p.H * 128;
     g.tiles_n = g.N / kFaBN;
     g.chunks = K / kFaBK;
     g.qkv.qo = p.qo;
