@@ -70,6 +70,10 @@ size_t attention_scratch_bytes(int B, int S_q, int Bk, int S_kv, int H, int D, A
 }
 
 namespace {
+// A row pass over the queries of a small grid, with the gap before it (256
+// tokens, B = 2, H = 16).
+constexpr float kRowPassUs = 6.0f;
+
 const FlashTimes &times_of(AttnMode mode)
 {
     return mode == kAttnBF16 ? kTimesBF16 : mode == kAttnF32X3 ? kTimesX3 : kTimesF32;
@@ -147,6 +151,17 @@ bool prepare_kv(const float *k, const float *v, const float *k_norm_w, const flo
            prepare_v(v, v_out, Bk, S_kv, H, D, mode, st);
 }
 
+bool attention_takes_q_planes(int B, int S_q, int S_kv, int H, int D, AttnMode mode,
+                              size_t balance_bytes)
+{
+    FlashScratch scr;
+    scr.part_bytes = flash_split_bytes(int64_t(B) * H, S_q, S_kv, D);
+    scr.balance_bytes = balance_bytes;
+    scr.keys = mode != kAttnF32;
+    scr.keys_saves = kRowPassUs;
+    return flash_plan(int64_t(B) * H, S_q, S_kv, D, times_of(mode), false, scr).keys;
+}
+
 bool run_attention(const AttnInputs &in, void *scratch, hipStream_t st)
 {
     const int B = in.B, S_q = in.S_q, S_kv = in.S_kv, H = in.H, D = in.D;
@@ -222,6 +237,7 @@ bool run_attention(const AttnInputs &in, void *scratch, hipStream_t st)
     FlashScratch scr;
     scr.part = cur;
     scr.part_bytes = flash_split_bytes(int64_t(B) * H, S_q, S_kv, D);
+    scr.keys = mode != kAttnF32;
     if (in.balance && (reinterpret_cast<uintptr_t>(in.balance) & 15u) == 0) {
         scr.balance = in.balance;
         scr.balance_bytes = in.balance_bytes;
@@ -246,12 +262,19 @@ bool run_attention(const AttnInputs &in, void *scratch, hipStream_t st)
     const auto a16 = [](const void *x) { return (reinterpret_cast<uintptr_t>(x) & 15u) == 0; };
     // A dealt workgroup of a balanced grid repeats it for its second part, as
     // it repeats the query load.
-    const FlashPlan raw_plan = flash_plan(int64_t(B) * H, S_q, S_kv, D, times_of(mode), false,
-                                          scr.part_bytes, scr.balance_bytes);
-    const bool raw_kernel =
-        mode == kAttnBF16 ? flash_bf16_raw_q(raw_plan, S_kv) : raw_plan.waves == 8;
-    const bool raw_q = !q_ready && prepared && !in.freqs && D == 128 && a16(in.q) &&
-                       ld_q % 4 == 0 && (!in.q_norm_w || a16(in.q_norm_w)) && raw_kernel;
+    // The keys shape takes raw rows too, once for all its key groups, and as
+    // the planes of a split-K product.
+    const bool raw_ok = !q_ready && prepared && !in.freqs && D == 128 && a16(in.q) &&
+                        ld_q % 4 == 0 && (!in.q_norm_w || a16(in.q_norm_w));
+    if (raw_ok)
+        scr.keys_saves = kRowPassUs;
+    const FlashPlan raw_plan =
+        flash_plan(int64_t(B) * H, S_q, S_kv, D, times_of(mode), false, scr);
+    const bool raw_kernel = raw_plan.keys || (mode == kAttnBF16 ? flash_bf16_raw_q(raw_plan, S_kv)
+                                                               : raw_plan.waves == 8);
+    const bool raw_q = raw_ok && raw_kernel;
+    if (in.q_parts > 1 && !(raw_q && raw_plan.keys))
+        return fail("attention: query planes need the keys shape");
 
     // Q rows, and K rows unless prepared, in one launch.
     const RowProblem pq =
@@ -286,6 +309,8 @@ bool run_attention(const AttnInputs &in, void *scratch, hipStream_t st)
         p.rq.s = bshd(S_q, H, D, false, in.ld_q);
         p.rq.w = in.q_norm_w;
         p.rq.eps = in.eps;
+        p.rq.parts = in.q_parts;
+        p.rq.plane = in.q_plane;
     }
     if (in.out_t) {
         p.o = nullptr;

@@ -47,6 +47,10 @@ struct RawQ {
     const float *w = nullptr;
     const float *freqs = nullptr;
     float eps = 1e-6f;
+    // The rows as the sum of `parts` planes, `plane` elements apart, added in
+    // order (the keys shape; 1 elsewhere).
+    int parts = 1;
+    int64_t plane = 0;
 };
 
 // Everything the attention kernels need; pointers are device pointers.
@@ -64,7 +68,7 @@ bool term_out_ok(const TermOut &t);  // alignment of a set term output
 
 // Launch shape of the D == 128 flash kernels: T = B*H*ceil(S_q/256) query
 // tiles of 8-wave workgroups, or twice as many of 4 waves, over n key tiles of
-// 64 keys, on 256 CUs that hold one workgroup each.  Four shapes:
+// 64 keys, on 256 CUs that hold one workgroup each.  Five shapes:
 //   whole     8-wave workgroups, one query tile each;
 //   small     4-wave workgroups, one query tile each (T < 256);
 //   split     4-wave workgroups, the key range of every query tile split over
@@ -73,10 +77,13 @@ bool term_out_ok(const TermOut &t);  // alignment of a set term output
 //   balanced  the largest multiple of 256 query tiles whole, and the key tiles
 //             of the `ntail` others as one list dealt out evenly, `u` to each
 //             of the last workgroups (T = 288 over 36 key tiles: 36 + 5 tiles
+//   keys      (bf16 MFMA) 8-wave workgroups of 64 query rows whose waves share
+//             the keys among them (flash_keys.hip): at most 256 of them.
 // A workgroup that sees part of a query tile's keys writes its output
 // normalised by its own row sum, plus that row's (max, sum), to scratch, and
 // flash_combine merges the parts into O.
 struct FlashPlan {
+    bool keys = false;    // the keys shape
     int waves = 8;
     int splits = 1;
     int tiles = 1 << 30;  // key tiles per split
@@ -93,20 +100,37 @@ struct FlashPlan {
 // round of at most about 0.7 of the CUs clocks higher, down to `part` of w8
 // (x3, T = 288 .. 800: 0.66 .. 0.76 of the full rounds' time per tile); the
 // f32 MFMA runs at full clock either way.
+// The keys shape: `round` for every 64 KiB of K that its four key groups take
+// together (keys_round of them), and `merge` once, both against what a 4-wave
+// workgroup spends beside its tiles (256 and 1024 queries and keys, 16 heads;
+// 0: the mode has no such kernel).
 struct FlashTimes {
-    float w4, w8, part;
+    float w4, w8, part, merge, round;
+    int keys_round;
 };
-constexpr FlashTimes kTimesF32{9.1f, 15.7f, 1.0f}, kTimesBF16{1.3f, 1.9f, 0.7f},
-    kTimesX3{2.5f, 4.6f, 0.7f};
+constexpr FlashTimes kTimesF32{9.1f, 15.7f, 1.0f, 0.0f, 0.0f, 0},
+    kTimesBF16{1.3f, 1.9f, 0.7f, 1.5f, 2.8f, 256}, kTimesX3{2.5f, 4.6f, 0.7f, 1.0f, 3.2f, 128};
 // Fixed cost (us) of split grids and of balanced ones, whose parts are twice
 // as tall: every part loads its query tile and writes f32 partials, which the
 // combine pass reads back (25 to 31 us at T = 144 and 288, every mode).
 constexpr float kSplitCostUs = 13.0f, kBalanceCostUs = 27.0f;
+// Scratch a flash launch may use, 16-byte aligned; either may be null.
+struct FlashScratch {
+    void *part = nullptr;
+    size_t part_bytes = 0;
+    void *balance = nullptr;
+    size_t balance_bytes = 0;
+    bool keys = false;  // the keys shape may run (the caller needs no other shape's bits)
+    // What it saves (us) because it alone takes the query rows raw: a row pass
+    // of its own before the kernel.
+    float keys_saves = 0.0f;
+};
+
 // The shape with the least predicted time among those whose partials fit:
-// part_bytes of scratch for `split`, balance_bytes for `balanced` (causal
-// calls, whose tiles differ in length, are not balanced).
+// s.part_bytes for `split`, s.balance_bytes for `balanced` (causal calls, whose
+// tiles differ in length, are not balanced, and `keys` has no mask).
 FlashPlan flash_plan(int64_t BH, int S_q, int S_kv, int D, const FlashTimes &t, bool causal,
-                     size_t part_bytes, size_t balance_bytes);
+                     const FlashScratch &s);
 // Scratch that holds the partials of a split grid in every mode, and that of
 // a balanced grid (0 where none would run).
 size_t flash_split_bytes(int64_t BH, int S_q, int S_kv, int D);
@@ -114,14 +138,6 @@ size_t flash_balance_bytes(int64_t BH, int S_q, int S_kv, int D, const FlashTime
 constexpr size_t kMaxFlashBalanceBytes = size_t(511) * 256 * (128 * 4 + 8);  // 65 MiB
 // A grid of 8-wave workgroups with at least one for each CU.
 bool flash_fills_gpu(int64_t BH, int S_q, int D);
-
-// Scratch a flash launch may use, 16-byte aligned; either may be null.
-struct FlashScratch {
-    void *part = nullptr;
-    size_t part_bytes = 0;
-    void *balance = nullptr;
-    size_t balance_bytes = 0;
-};
 
 // What a workgroup that sees part of the keys writes (device view).  Partials
 // of a split grid are laid out [splits][BH][S_q][128] f32 and (max, sum) pairs
@@ -148,6 +164,9 @@ bool launch_flash_combine(const FlashProblem &p, const FlashSplitArgs &sa, hipSt
 
 // f32 inputs, f32 MFMA (D == 128) or the generic kernel (any D <= 1024).
 bool launch_flash_f32(const FlashProblem &p, hipStream_t st, const FlashScratch &scr = {});
+// The keys shape of the bf16 (terms 1) and f32x3 (2) kernels, on operands their
+// launchers checked (flash_keys.hip).
+bool launch_flash_keys(const FlashProblem &p, int terms, bool dma32, hipStream_t st);
 // True when launch_flash_f32 would take the MFMA path for this problem.
 bool flash_f32_fast_path(const FlashProblem &p);
 
@@ -350,6 +369,10 @@ enum AttnMode : int { kAttnF32 = 0, kAttnBF16 = 1, kAttnF32X3 = 2 };
 // [Bk, H, 2D, vt_padded_len(S_kv)].
 struct AttnInputs {
     const float *q = nullptr;         // [B, S_q, H, D] f32 projections
+    // q as the sum of q_parts planes q_plane elements apart (prepared K/V, 16-byte
+    // alignment, and a shape attention_takes_q_planes() says yes to).
+    int q_parts = 1;
+    int64_t q_plane = 0;
     const float *q_norm_w = nullptr;  // [D] or null
     const float *freqs = nullptr;     // [S_q, D/2, 2, 2] or null (self-attention)
     const float *k = nullptr;         // raw [Bk, S_kv, H, D] f32 (when not prepared)
@@ -433,6 +456,8 @@ void use_balance_scratch(AttnInputs &in, void *scratch, size_t scratch_bytes, si
 bool prepare_kv(const float *k, const float *v, const float *k_norm_w, const float *freqs,
                 void *k_out, void *v_out, int Bk, int S_kv, int H, int D, float eps,
                 AttnMode mode, hipStream_t st);
+bool attention_takes_q_planes(int B, int S_q, int S_kv, int H, int D, AttnMode mode,
+                              size_t balance_bytes);
 bool run_attention(const AttnInputs &in, void *scratch, hipStream_t st);
 
 // ---- Attention sub-block of a DiT block on the resident residual stream

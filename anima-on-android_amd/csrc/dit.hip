@@ -763,9 +763,22 @@ bool dit_sublayer(const anima_hip_dit *d, const BlockWeights &bw, int kind, floa
         in.Bk = B;
         in.S_kv = int(S);
     } else {
-        if (!dit_product(d, terms, d->ld_d, bw.w_cq, d->ld_d, proj, HD, M, rws, l.ws, st))
-            return false;
-        in.q = proj;
+        // Where the small-M GEMM splits K and the attention adds up query
+        // planes itself, q stays in its partial planes: no reduction pass.
+        if (d->reps == 2 && l.ws >= size_t(M) * HD * 4 && c.head_dim == 128 && aligned16(bw.cx_qn) &&
+            attention_takes_q_planes(B, int(S), d->ctx_S, c.heads, c.head_dim, d->attn,
+                                     balance_bytes)) {
+            in.q = reinterpret_cast<float *>(rws);
+            in.q_plane = M * HD;
+            if (!launch_linear_planes(terms, d->ld_d, int(d->ld_d / 2), true, bw.w_cq, d->ld_d,
+                                      reinterpret_cast<float *>(rws), l.ws, int(M), HD,
+                                      &in.q_parts, st))
+                return false;
+        } else {
+            if (!dit_product(d, terms, d->ld_d, bw.w_cq, d->ld_d, proj, HD, M, rws, l.ws, st))
+                return false;
+            in.q = proj;
+        }
         in.q_norm_w = bw.cx_qn;
         in.k_prep = bw.ctx_k;
         in.v_prep = bw.ctx_v;

@@ -486,8 +486,7 @@ bool launch_flash_f32(const FlashProblem &p, hipStream_t st, const FlashScratch 
         a.raw_q = raw_q ? 1 : 0;
         a.qw = p.rq.w;
         a.eps = p.rq.eps;
-        const FlashPlan pl = flash_plan(BH, p.S_q, p.S_kv, p.D, kTimesF32, p.causal,
-                                        scr.part_bytes, scr.balance_bytes);
+        const FlashPlan pl = flash_plan(BH, p.S_q, p.S_kv, p.D, kTimesF32, p.causal, scr);
         FlashDeal deal;
         a.split = flash_split_args(pl, BH, p.S_q, scr, deal);
         if (!(pl.waves == 4 ? launch_d128<4>(a, FlashWhole{}, BH, st)

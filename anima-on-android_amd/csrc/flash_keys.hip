@@ -1,0 +1,387 @@
+// Flash attention for grids that leave most of the GPU idle: a workgroup's
+// waves share the keys of 64 query rows (gfx950, bf16 MFMA, D = 128).
+//
+// The computation, operands and layouts of flash_bf16.hip (TERMS = 1: bf16 q
+// and k rows, packed V^T) and flash_x3.hip (TERMS = 2: [hi | lo] term rows and
+// term V^T, every product as hi*hi + hi*lo + lo*hi); anima_rt_run_sdpa_flash
+// (anima_rt/src/anima_rt.cpp:147-156 -> anima_rt/include/cpu/flash_attention.h:
+// 55-208) without a mask.
+//
+// Why: those kernels give a wave 32 query rows and walk all keys in series, so
+// 256 queries of 16 heads are 32 workgroups of 4 waves on 256 CUs, each with
+// one wave per SIMD and every tile's latency in the open; split over more
+// workgroups they pay a combine pass.  Here 8 waves are 2 (query rows) x 4
+// (keys): wave (r, g) takes rows 32r .. 32r+31 and key tiles g, g + 4, ..., with
+// its own running max, sum and O; the four parts of a row are merged through
+// LDS at the end.  Four times the workgroups, two waves per SIMD, no second
+// launch; each K/V tile serves 64 rows instead of 128 or 256, so the kernel is
+// bound by the L2 -> LDS stream (128 KiB per round of four tiles, about 35 bytes
+// per clock and CU) where the grid fills the GPU.
+// Whole attention calls on MI355X before and now, 16 heads (f32x3 / bf16): self
+// 256 tokens 24.7 -> 22.5 / 17.8 -> 16.4 us, 1024 tokens 50.4 -> 46.6 / 39.1 ->
+// 30.8; cached cross-attention, query rows normalised in here, 256 x 512
+// 28.8 -> 23.1 / 20.7 -> 16.8, 1024 x 512 34.5 -> 24.6 / 22.6 -> 17.9.  A round
+// takes about 4 us (f32x3): each of its two phases waits for 64 KiB of copies.
+//
+// Per key group one K tile and one V^T tile (16 KiB each: 32 keys of terms, 64
+// of bf16), single-buffered and refilled in turn: V^T lands while the scores
+// run, the next K while the softmax and P.V run, one barrier after each.
+#include "qrow.h"
+
+#include <cmath>
+
+namespace anima_hip {
+namespace {
+
+using namespace flash_tile;
+
+constexpr int kGroups = 4;           // key groups of a workgroup
+constexpr int kRowsPerBlock = 64;    // query rows of a workgroup
+constexpr int kTileEl = 8192;        // bf16 per K or V^T tile (16 KiB)
+constexpr int kPitch = kD + 4;       // floats per merged row (4 against bank conflicts)
+constexpr int kRingBytes = kGroups * 2 * kTileEl * 2;
+constexpr int kMergeBytes = 8 * 32 * kPitch * 4;
+
+struct KeysArgs {
+    const u16 *q, *k, *vt;
+    float *o;
+    int64_t qb, qh, qs, kb, kh, ks, vb, vh, vd, ob, oh, os;
+    int H, S_q, S_kv, n_qtiles;
+    float c;    // scale * log2(e), > 0
+    int dma32;  // K/V^T tile rows fit 32-bit byte offsets from the tile start
+    TermOut ot;
+    const float *qx, *qw, *qf;  // raw query rows (RawQ) in place of q when qx is set
+    int64_t rqb, rqh, rqs, qplane;
+    int qparts;
+    float eps;
+};
+
+// A part with any sum but zero takes part in the merge, a NaN sum included (by
+// bits: this file is compiled without NaN comparisons).
+__device__ __forceinline__ bool joins(const float2 &p) { return (__float_as_uint(p.y) << 1) != 0; }
+
+template <int TERMS>
+__global__ __launch_bounds__(512, 1) void flash_keys_d128(KeysArgs a)
+{
+    constexpr int KT = 64 / TERMS, NB = KT / 32;   // keys per tile, 32-key blocks
+    constexpr int kRow = TERMS * kD, CK = kRow / 8;  // K row: elements, 16-byte chunks
+    constexpr int CV = KT / 8;                     // chunks of a V^T row
+    constexpr int kCopies = kTileEl / 8 / 128;     // 16-byte copies per thread and tile
+    static_assert(KT * kRow == kTileEl, "tile sizes");
+    static_assert(kRowsPerBlock * kPitch * 4 <= kGroups * kTileEl * 2, "raw rows fit");
+
+    __shared__ __attribute__((aligned(16))) unsigned char
+        smem[kMergeBytes > kRingBytes ? kMergeBytes : kRingBytes];
+    __shared__ float2 ml[8][32];  // (max, sum) per wave and row
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 31, half = lane >> 5;
+    const int rg = wave & 1, kg = wave >> 1;
+    u16 *const ks = reinterpret_cast<u16 *>(smem) + kg * kTileEl;
+    u16 *const vs = ks + kGroups * kTileEl;
+
+    const int blk = xcd_major_block();
+    const int qt = blk % a.n_qtiles, bh = blk / a.n_qtiles;
+    const int b = bh / a.H, h = bh - b * a.H;
+    const int q0 = qt * kRowsPerBlock;
+    const int qrow = q0 + 32 * rg + col;
+    const u16 *kp = a.k + b * a.kb + h * a.kh;
+    const u16 *vp = a.vt + b * a.vb + h * a.vh;
+    const int ntiles = (a.S_kv + KT - 1) / KT;
+
+    // Copy i of this wave fills the 64 chunks of window w = kCopies*rg + i of its
+    // group's tile.  LDS layouts, unpadded, XOR-swizzled so that the 16 lanes a
+    // fragment read serves per clock hit 16 bank groups: chunk c of K row r at
+    // c ^ (r & 15); of V^T row r at c ^ ((r >> 2) & 3) (four chunks a row) or
+    // c ^ ((r >> 1) & 7) (eight).
+    auto vswz = [](int r) { return TERMS == 2 ? (r >> 2) & 3 : (r >> 1) & 7; };
+    unsigned koff[kCopies], voff[2];
+#pragma unroll
+    for (int i = 0; i < kCopies; ++i) {
+        const int f = (kCopies * rg + i) * 64 + lane, r = f / CK;
+        koff[i] = unsigned(r * a.ks + 8 * ((f % CK) ^ (r & 15))) * 2u;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        // Rows of window i, from row (kCopies*rg) * 64/CV; the swizzle of a
+        // window depends on its parity only.
+        const int f = (kCopies * rg + i) * 64 + lane, r = f / CV;
+        voff[i] = unsigned((lane / CV) * a.vd + 8 * ((f % CV) ^ vswz(r))) * 2u;
+    }
+    auto dma_k = [&](int t) {
+        const int key0 = t * KT;
+        if (a.dma32 && key0 + KT <= a.S_kv) {
+#pragma unroll
+            for (int i = 0; i < kCopies; ++i)
+                dma16s(kp + int64_t(key0) * a.ks, koff[i], ks + (kCopies * rg + i) * 512);
+        } else {
+            // Keys past S_kv copy row S_kv - 1; their scores are masked.
+#pragma unroll
+            for (int i = 0; i < kCopies; ++i) {
+                const int f = (kCopies * rg + i) * 64 + lane, r = f / CK;
+                dma16(kp + int64_t(min(key0 + r, a.S_kv - 1)) * a.ks + 8 * ((f % CK) ^ (r & 15)),
+                      ks + (kCopies * rg + i) * 512);
+            }
+        }
+    };
+    auto dma_v = [&](int t) {
+        // V^T is zero-padded in HBM to whole 64-key tiles.
+        const u16 *base = vp + t * KT;
+#pragma unroll
+        for (int i = 0; i < kCopies; ++i) {
+            const int win = kCopies * rg + i;
+            if (a.dma32)
+                dma16s(base + int64_t(win * (64 / CV)) * a.vd, voff[i & 1], vs + win * 512);
+            else
+                dma16(base + int64_t(win * (64 / CV) + lane / CV) * a.vd +
+                          8 * (((win * 64 + lane) % CV) ^ vswz((win * 64 + lane) / CV)),
+                      vs + win * 512);
+        }
+    };
+    // Fragments: K key row col + 32*kb, term chunk 8*half + t; V^T row
+    // 128*term + 32*blk + col, keys [16i, 16i + 16) (chunk half + 2i).
+    auto kfrag = [&](int t, int kb, int term) {
+        return *reinterpret_cast<const bf16x8 *>(
+            ks + (col + 32 * kb) * kRow + 8 * (16 * term + (((half << 3) | t) ^ (col & 15))));
+    };
+    auto vfrag = [&](int blk, int i, int term) {
+        return *reinterpret_cast<const bf16x8 *>(vs + (128 * term + 32 * blk + col) * KT +
+                                                 8 * ((half + 2 * i) ^ vswz(col)));
+    };
+
+    if (kg < ntiles)
+        dma_k(kg);
+    // Q terms: hi Q[qrow][64*half + 8t .. +7], lo 128 elements further.
+    bf16x8 qh[8], ql[8];
+    if (a.qx) {
+        // The 64 raw rows once for the four key groups, through the V^T tiles'
+        // space, their planes added in order.
+        float *const rows = reinterpret_cast<float *>(smem + kGroups * kTileEl * 2);
+        f32x4 v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int f = tid + 512 * i, r = min(q0 + (f >> 5), a.S_q - 1);
+            const float *x = a.qx + b * a.rqb + h * a.rqh + int64_t(r) * a.rqs + 4 * (f & 31);
+            v[i] = *reinterpret_cast<const f32x4 *>(x);
+            for (int p = 1; p < a.qparts; ++p)
+                v[i] += *reinterpret_cast<const f32x4 *>(x + p * a.qplane);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int f = tid + 512 * i;
+            *reinterpret_cast<f32x4 *>(rows + (f >> 5) * kPitch + 4 * (f & 31)) = v[i];
+        }
+        __syncthreads();
+        q_terms_from_raw<TERMS == 2>(rows + (32 * rg + col) * kPitch, a.qw,
+                                     a.qf ? a.qf + int64_t(min(qrow, a.S_q - 1)) * 4 * kD / 2
+                                          : nullptr,
+                                     a.eps, true, half, qh, ql);
+    } else {
+        const u16 *qr = a.q + b * a.qb + h * a.qh + int64_t(min(qrow, a.S_q - 1)) * a.qs;
+        const bf16x8 *src = reinterpret_cast<const bf16x8 *>(qr + 64 * half);
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            qh[t] = src[t];
+            if (TERMS == 2)
+                ql[t] = src[kD / 8 + t];
+        }
+    }
+    f32x16 o[4] = {};
+    float m = -INFINITY, l = 0.0f, l2 = 0.0f;
+    wait_vmcnt<0>();
+    ring_barrier();
+
+    for (int t0 = 0; t0 < ntiles; t0 += kGroups) {
+        const int t = t0 + kg;  // this group's tile; none in a ragged last round
+        const bool live = t < ntiles;
+        f32x16 s[NB] = {};
+        if (live) {
+            dma_v(t);
+            // Scores S^T; with terms the cross products in a chain of their own.
+            f32x16 x = {};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+#pragma unroll
+                for (int kb = 0; kb < NB; ++kb) {
+                    const bf16x8 k0 = kfrag(i, kb, 0);
+                    s[kb] = mfma_bf16(k0, qh[i], s[kb]);
+                    if (TERMS == 2) {
+                        x = mfma_bf16(k0, ql[i], x);
+                        x = mfma_bf16(kfrag(i, kb, 1), qh[i], x);
+                    }
+                }
+            }
+            if (TERMS == 2)
+                s[0] += x;
+        }
+        wait_vmcnt<0>();
+        ring_barrier();  // V^T is there, K is read
+        if (t + kGroups < ntiles)
+            dma_k(t + kGroups);
+        if (live) {
+            const int key0 = t * KT;
+            if (key0 + KT > a.S_kv) {
+#pragma unroll
+                for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        if (key0 + 32 * kb + acc_row(r, half) >= a.S_kv)
+                            s[kb][r] = -INFINITY;
+            }
+            float mx = -INFINITY;
+#pragma unroll
+            for (int kb = 0; kb < NB; ++kb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    mx = fmaxf(mx, s[kb][r]);
+            // The max on raw scores (c > 0) and the lazy rescale, as in the
+            // kernels of whole key ranges.
+            const float cand = row_pair_max(mx) * a.c;
+            if (__any(cand > m + kRescaleLog2)) {
+                const float m_new = fmaxf(m, cand);
+                const float alpha =
+                    m_new == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - m_new);
+                m = m_new;
+                l *= alpha;
+                l2 *= alpha;
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+                    o[d] *= alpha;
+            }
+            const float neg_m = (m == -INFINITY) ? 0.0f : -m;
+            // P in chunks of 16 keys, its terms summed as the MFMAs take them.
+            float sum = 0.0f, sum2 = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 2 * NB; ++i) {
+                f32x16 &sc = s[i >> 1];
+                bf16x8 ph, pl;
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    sc[8 * (i & 1) + e] =
+                        __builtin_amdgcn_exp2f(fmaf(sc[8 * (i & 1) + e], a.c, neg_m));
+                ph = pack8(sc, 8 * (i & 1));
+                sum = row_sum8(ph, sum);
+                if (TERMS == 2) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        sc[8 * (i & 1) + e] -= float(ph[e]);
+                    pl = pack8(sc, 8 * (i & 1));
+                    sum2 = row_sum8(pl, sum2);
+                }
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    const bf16x8 v0 = vfrag(d, i, 0);
+                    o[d] = mfma_bf16(v0, ph, o[d]);
+                    if (TERMS == 2) {
+                        o[d] = mfma_bf16(v0, pl, o[d]);
+                        o[d] = mfma_bf16(vfrag(d, i, 1), ph, o[d]);
+                    }
+                }
+            }
+            l += sum;
+            l2 += sum2;
+        }
+        wait_vmcnt<0>();
+        ring_barrier();  // the next K is there, V^T is read
+    }
+
+    // Merge the four parts of every row: a part whose max never left -inf saw
+    // masked or NaN scores only and drops out; a NaN sum joins and makes the
+    // row NaN, as in the reference.
+    l += l2;
+    l += __shfl_xor(l, 32);
+    if (half == 0)
+        ml[wave][col] = make_float2(m, m == -INFINITY ? 0.0f : l);
+    __syncthreads();
+    float mx = -INFINITY;
+#pragma unroll
+    for (int g = 0; g < kGroups; ++g) {
+        const float2 p = ml[2 * g + rg][col];
+        if (joins(p))
+            mx = fmaxf(mx, p.x);
+    }
+    const float w = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
+    float *const part = reinterpret_cast<float *>(smem);
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            f32x4 v = f32x4{o[d][4 * g], o[d][4 * g + 1], o[d][4 * g + 2], o[d][4 * g + 3]} * w;
+            if (m == -INFINITY)
+                v = f32x4{0.f, 0.f, 0.f, 0.f};
+            *reinterpret_cast<f32x4 *>(part + (wave * 32 + col) * kPitch + 32 * d +
+                                       acc_row(4 * g, half)) = v;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < kRowsPerBlock * 32 / 512; ++i) {
+        const int f = tid + 512 * i, r = f >> 5, c4 = f & 31;
+        if (q0 + r >= a.S_q)
+            continue;
+        const int r0 = r >> 5, rr = r & 31;
+        float top = -INFINITY;
+#pragma unroll
+        for (int g = 0; g < kGroups; ++g) {
+            const float2 p = ml[2 * g + r0][rr];
+            if (joins(p))
+                top = fmaxf(top, p.x);
+        }
+        float sum = 0.0f;
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int g = 0; g < kGroups; ++g) {
+            const float2 p = ml[2 * g + r0][rr];
+            if (joins(p)) {
+                sum += p.y * __builtin_amdgcn_exp2f(p.x - top);
+                v += *reinterpret_cast<const f32x4 *>(part + ((2 * g + r0) * 32 + rr) * kPitch +
+                                                      4 * c4);
+            }
+        }
+        v *= sum > 0.0f ? 1.0f / sum : 0.0f;  // a NaN sum has NaN in v
+        const int q = q0 + r;
+        store_out4(v, a.o + b * a.ob + h * a.oh + int64_t(q) * a.os,
+                   a.ot.t ? a.ot.t + b * a.ot.tb + h * a.ot.th + int64_t(q) * a.ot.ts : nullptr,
+                   a.ot.lo, 4 * c4);
+    }
+}
+
+}  // namespace
+
+bool launch_flash_keys(const FlashProblem &p, int terms, bool dma32, hipStream_t st)
+{
+    const int64_t BH = int64_t(p.B) * p.H;
+    KeysArgs a;
+    a.q = static_cast<const u16 *>(p.q);
+    a.k = static_cast<const u16 *>(p.k);
+    a.vt = static_cast<const u16 *>(p.v);
+    a.o = p.o;
+    a.qb = p.qs.b; a.qh = p.qs.h; a.qs = p.qs.s;
+    a.kb = p.ks.b; a.kh = p.ks.h; a.ks = p.ks.s;
+    a.vb = p.vs.b; a.vh = p.vs.h; a.vd = vt_padded_len(p.S_kv);
+    a.ob = p.os.b; a.oh = p.os.h; a.os = p.os.s;
+    a.H = p.H;
+    a.S_q = p.S_q;
+    a.S_kv = p.S_kv;
+    a.n_qtiles = (p.S_q + kRowsPerBlock - 1) / kRowsPerBlock;
+    a.c = p.scale * kLog2e;
+    a.dma32 = dma32 ? 1 : 0;
+    a.ot = p.ot;
+    a.qx = p.rq.x;
+    a.qw = p.rq.w;
+    a.qf = p.rq.freqs;
+    a.rqb = p.rq.s.b; a.rqh = p.rq.s.h; a.rqs = p.rq.s.s;
+    a.qparts = p.rq.parts;
+    a.qplane = p.rq.plane;
+    a.eps = p.rq.eps;
+    const int64_t nblk = BH * a.n_qtiles;
+    if (nblk > INT32_MAX)
+        return fail("flash_keys: problem too large for one launch");
+    if (terms == 2)
+        hipLaunchKernelGGL(flash_keys_d128<2>, dim3(unsigned(nblk)), dim3(512), 0, st, a);
+    else
+        hipLaunchKernelGGL(flash_keys_d128<1>, dim3(unsigned(nblk)), dim3(512), 0, st, a);
+    return hip_ok(hipGetLastError(), "flash_keys_d128 launch");
+}
+
+}  // namespace anima_hip

@@ -174,7 +174,7 @@ FlashPlan balanced_plan(int64_t BH, int S_q, int S_kv, int D)
 }  // namespace
 
 FlashPlan flash_plan(int64_t BH, int S_q, int S_kv, int D, const FlashTimes &t, bool causal,
-                     size_t part_bytes, size_t balance_bytes)
+                     const FlashScratch &s)
 {
     FlashPlan best;
     if (D != kD || BH <= 0 || S_q <= 0)
@@ -197,12 +197,21 @@ FlashPlan flash_plan(int64_t BH, int S_q, int S_kv, int D, const FlashTimes &t, 
         small.waves = 4;
         consider(small, rounds(T4) * n * t.w4);
         const FlashPlan sp = split_plan(BH, S_q, S_kv, D);
-        if (sp.splits > 1 && sp.bytes <= part_bytes)
+        if (sp.splits > 1 && sp.bytes <= s.part_bytes)
             consider(sp, rounds(T4 * sp.splits) * sp.tiles * t.w4 + kSplitCostUs);
     }
     const FlashPlan bal = balanced_plan(BH, S_q, S_kv, D);
-    if (bal.u > 0 && !causal && bal.bytes <= balance_bytes)
+    if (bal.u > 0 && !causal && bal.bytes <= s.balance_bytes)
         consider(bal, (bal.full / kTargetBlocks * n + bal.u) * t.w8 + kBalanceCostUs);
+    // One key tile of 64 has nothing to share (64 queries and keys, 16 heads:
+    // 14.1 us whole against 16.1), and a second round of workgroups loses to
+    // the taller tiles (576 queries and keys, 32 heads, f32x3: 46 against 60).
+    if (s.keys && t.keys_round > 0 && !causal && S_kv > kBN &&
+        BH * ceil_div(S_q, 64) <= kTargetBlocks) {
+        FlashPlan keys;
+        keys.keys = true;
+        consider(keys, t.merge + ceil_div(S_kv, t.keys_round) * t.round - s.keys_saves);
+    }
     return best;
 }
 
@@ -213,7 +222,9 @@ size_t flash_split_bytes(int64_t BH, int S_q, int S_kv, int D)
 
 size_t flash_balance_bytes(int64_t BH, int S_q, int S_kv, int D, const FlashTimes &t)
 {
-    const FlashPlan pl = flash_plan(BH, S_q, S_kv, D, t, false, SIZE_MAX, SIZE_MAX);
+    FlashScratch any;
+    any.part_bytes = any.balance_bytes = SIZE_MAX;
+    const FlashPlan pl = flash_plan(BH, S_q, S_kv, D, t, false, any);
     return pl.u > 0 ? pl.bytes : 0;
 }
 

@@ -520,8 +520,11 @@ bool launch_flash_x3(const FlashProblem &p, hipStream_t st, const FlashScratch &
     a.qf = p.rq.freqs;
     a.rqb = p.rq.s.b; a.rqh = p.rq.s.h; a.rqs = p.rq.s.s;
     a.eps = p.rq.eps;
-    const FlashPlan pl = flash_plan(BH, p.S_q, p.S_kv, p.D, kTimesX3, p.causal, scr.part_bytes,
-                                    scr.balance_bytes);
+    const FlashPlan pl = flash_plan(BH, p.S_q, p.S_kv, p.D, kTimesX3, p.causal, scr);
+    if (pl.keys)
+        return launch_flash_keys(p, 2, a.dma32 != 0, st);
+    if (p.rq.parts > 1)
+        return fail("flash_x3: this launch shape takes no query planes");
     FlashDeal deal;
     a.split = flash_split_args(pl, BH, p.S_q, scr, deal);
     if (!(pl.waves == 4 ? launch_d128<4>(a, FlashWhole{}, BH, st)
