@@ -74,9 +74,14 @@ struct LnArgs {
 
 // Row r of batch entry r / S, spread over WPR waves of the 4-wave block (4 /
 // WPR rows per block): wave w takes the float4 columns c = 64 (w % WPR) +
-// lane + 64 WPR i, i < VPL, so VPL float4 per lane cover Dm <= 256 WPR VPL.  Every load of the row (x, the
-// pending residual's planes, the gate) is issued before the first store.
-template <int VPL, int WPR>
+// lane + 64 WPR i, i < VPL, so VPL float4 per lane cover Dm <= 256 WPR VPL.
+// Every load of the row (x, the pending residual, the gate) is issued before
+// the first store.
+// Bound by HBM.  PLANES: the pending residual is several planes, at small M,
+// where latency shows; then the modulation too is loaded ahead of the row sums,
+// and the planes four at a time (512 rows of 2048, four planes: 8.7 -> 8.0 us;
+// at 2048 rows of one plane the earlier loads measured 1 % slower).
+template <int VPL, int WPR, bool PLANES>
 __global__ __launch_bounds__(256) void ln_modulate_kernel(LnArgs a)
 {
     constexpr int RPB = 4 / WPR;  // rows per block
@@ -86,7 +91,7 @@ __global__ __launch_bounds__(256) void ln_modulate_kernel(LnArgs a)
     const int64_t row = int64_t(blockIdx.x) * RPB + wave / WPR;
     const bool live = row < a.M;  // uniform per row group (the barriers need every wave)
     const int64_t r = live ? row : 0;
-    const int b = int(r / a.S);
+    const int b = int(unsigned(r) / unsigned(a.S));
     const float *x = a.x + r * a.ldx;
     const int n4 = a.Dm >> 2;
     f32x4 v[VPL];
@@ -97,6 +102,21 @@ __global__ __launch_bounds__(256) void ln_modulate_kernel(LnArgs a)
         v[i] = c < n4 && live ? *reinterpret_cast<const f32x4 *>(x + 4 * c)
                               : f32x4{0.f, 0.f, 0.f, 0.f};
     }
+    const float *shift = a.mod + int64_t(b) * a.mod_ld;
+    const float *scale = shift + a.Dm;
+    f32x4 sh[VPL], sc[VPL];
+    auto load_mod = [&] {
+#pragma unroll
+        for (int i = 0; i < VPL; ++i) {
+            const int c = 64 * seg + lane + 64 * WPR * i;
+            if (c < n4) {
+                sh[i] = *reinterpret_cast<const f32x4 *>(shift + 4 * c);
+                sc[i] = *reinterpret_cast<const f32x4 *>(scale + 4 * c);
+            }
+        }
+    };
+    if (PLANES)
+        load_mod();
     if (a.res_y && live) {
         const float *yr = a.res_y + r * a.Dm;
         const float *gr = a.res_gate + b * a.res_ld;
@@ -109,13 +129,25 @@ __global__ __launch_bounds__(256) void ln_modulate_kernel(LnArgs a)
                 g[i] = *reinterpret_cast<const f32x4 *>(gr + 4 * c);
             }
         }
-        for (int p = 1; p < a.res_parts; ++p) {
+        for (int p0 = 1; PLANES && p0 < a.res_parts; p0 += 3) {
+            f32x4 t[3][VPL];
 #pragma unroll
-            for (int i = 0; i < VPL; ++i) {
-                const int c = 64 * seg + lane + 64 * WPR * i;
-                if (c < n4)
-                    y[i] += *reinterpret_cast<const f32x4 *>(yr + p * a.res_plane + 4 * c);
+            for (int u = 0; u < 3; ++u) {
+                const int p = min(p0 + u, a.res_parts - 1);  // past the last: read, not added
+#pragma unroll
+                for (int i = 0; i < VPL; ++i) {
+                    const int c = 64 * seg + lane + 64 * WPR * i;
+                    if (c < n4)
+                        t[u][i] = *reinterpret_cast<const f32x4 *>(yr + p * a.res_plane + 4 * c);
+                }
             }
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+                if (p0 + u < a.res_parts) {
+#pragma unroll
+                    for (int i = 0; i < VPL; ++i)
+                        y[i] += t[u][i];
+                }
         }
 #pragma unroll
         for (int i = 0; i < VPL; ++i) {
@@ -156,17 +188,16 @@ __global__ __launch_bounds__(256) void ln_modulate_kernel(LnArgs a)
     const float rstd = 1.0f / sqrtf(row_sum(sq, 1) / float(a.Dm) + a.eps);
     if (!live)
         return;
-    const float *shift = a.mod + int64_t(b) * a.mod_ld;
-    const float *scale = shift + a.Dm;
+    if (!PLANES)
+        load_mod();
     if (a.yf) {
 #pragma unroll
         for (int i = 0; i < VPL; ++i) {
             const int c = 64 * seg + lane + 64 * WPR * i;
             if (c < n4) {
-                const f32x4 sc = *reinterpret_cast<const f32x4 *>(scale + 4 * c);
-                const f32x4 sh = *reinterpret_cast<const f32x4 *>(shift + 4 * c);
                 const f32x4 xn = (v[i] - mean) * rstd;
-                *reinterpret_cast<f32x4 *>(a.yf + r * a.ldy + 4 * c) = xn * (1.0f + sc) + sh;
+                *reinterpret_cast<f32x4 *>(a.yf + r * a.ldy + 4 * c) =
+                    xn * (1.0f + sc[i]) + sh[i];
             }
         }
         return;
@@ -177,10 +208,8 @@ __global__ __launch_bounds__(256) void ln_modulate_kernel(LnArgs a)
     for (int i = 0; i < VPL; ++i) {
         const int c = 64 * seg + lane + 64 * WPR * i;
         if (c < n4) {
-            const f32x4 sc = *reinterpret_cast<const f32x4 *>(scale + 4 * c);
-            const f32x4 sh = *reinterpret_cast<const f32x4 *>(shift + 4 * c);
             const f32x4 xn = (v[i] - mean) * rstd;
-            const f32x4 y = xn * (1.0f + sc) + sh;
+            const f32x4 y = xn * (1.0f + sc[i]) + sh[i];
             const unsigned int h0 = pack_pair(y.x, y.y), h1 = pack_pair(y.z, y.w);
             *reinterpret_cast<uint2 *>(hrow + 2 * c) = uint2{h0, h1};
             if (lrow) {
@@ -306,12 +335,14 @@ bool launch_ln_modulate(const float *x, int64_t ldx, const float *mod, int64_t m
         return fail("ln_modulate: too many rows");
     const int vpl = (Dm + 256 * wpr - 1) / (256 * wpr);
     const dim3 grid{unsigned(nblk)}, block{256};
-    if (vpl <= 1)
-        hipLaunchKernelGGL((ln_modulate_kernel<1, wpr>), grid, block, 0, st, a);
-    else if (vpl <= 2)
-        hipLaunchKernelGGL((ln_modulate_kernel<2, wpr>), grid, block, 0, st, a);
-    else
-        hipLaunchKernelGGL((ln_modulate_kernel<4, wpr>), grid, block, 0, st, a);
+    const bool planes = res_y && res_parts > 1;
+    const auto run = planes ? vpl <= 1   ? ln_modulate_kernel<1, wpr, true>
+                              : vpl <= 2 ? ln_modulate_kernel<2, wpr, true>
+                                         : ln_modulate_kernel<4, wpr, true>
+                     : vpl <= 1 ? ln_modulate_kernel<1, wpr, false>
+                     : vpl <= 2 ? ln_modulate_kernel<2, wpr, false>
+                                : ln_modulate_kernel<4, wpr, false>;
+    hipLaunchKernelGGL(run, grid, block, 0, st, a);
     return hip_ok(hipGetLastError(), "ln_modulate_kernel launch");
 }
 

@@ -158,14 +158,29 @@ __global__ __launch_bounds__(512, 1) void flash_keys_d128(KeysArgs a)
         // The 64 raw rows once for the four key groups, through the V^T tiles'
         // space, their planes added in order.
         float *const rows = reinterpret_cast<float *>(smem + kGroups * kTileEl * 2);
+        const float *x[4];
         f32x4 v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int f = tid + 512 * i, r = min(q0 + (f >> 5), a.S_q - 1);
-            const float *x = a.qx + b * a.rqb + h * a.rqh + int64_t(r) * a.rqs + 4 * (f & 31);
-            v[i] = *reinterpret_cast<const f32x4 *>(x);
-            for (int p = 1; p < a.qparts; ++p)
-                v[i] += *reinterpret_cast<const f32x4 *>(x + p * a.qplane);
+            x[i] = a.qx + b * a.rqb + h * a.rqh + int64_t(r) * a.rqs + 4 * (f & 31);
+            v[i] = *reinterpret_cast<const f32x4 *>(x[i]);
+        }
+        for (int p0 = 1; p0 < a.qparts; p0 += 3) {  // three planes' loads in flight
+            f32x4 y[3][4];
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)  // past the last plane: read, not added
+                    y[u][i] = *reinterpret_cast<const f32x4 *>(
+                        x[i] + min(p0 + u, a.qparts - 1) * a.qplane);
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+                if (p0 + u < a.qparts) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        v[i] += y[u][i];
+                }
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
