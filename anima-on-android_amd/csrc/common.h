@@ -222,6 +222,9 @@ size_t linear_scratch_bytes(int M, int K, bool exact);
 bool launch_linear(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, float *c,
                    int64_t ldc, int M, int N, int K, bool exact, void *scratch,
                    size_t scratch_bytes, hipStream_t st);
+// launch_linear (exact) runs this shape on gemm_f32a.hip.
+bool linear_takes_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, const float *c,
+                       int64_t ldc, int M, int N, int K);
 
 // A split into [hi | lo] rows of 2*linear_terms_ld(K) bf16 (the product with
 // a weight whose rows are [W | W], K' = 2 * linear_terms_ld(K), is then one
@@ -251,12 +254,18 @@ bool gemm_large_f32a_supported(int M, int N, int K, int64_t lda, int64_t ldw, in
                                const float *a, const void *w, const void *c);
 bool launch_gemm_large_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, float *c,
                             int64_t ldc, int M, int N, int K, hipStream_t st);
-// Large-M product on f32 activations in 256 x 256 tiles (gemm_f32a.hip): a
-// [M][lda] (lda % 4 == 0, K % 32 == 0) split into bf16 hi + lo terms
-// (two_terms) or rounded to bf16 in registers, C f32.  With two terms C is
-// bit-identical to the split pass plus launch_gemm_large on the term rows.
+// Product on f32 activations (gemm_f32a.hip): a [M][lda] (lda % 4 == 0, K % 32
+// == 0) split into bf16 hi + lo terms (two_terms; tiles of 256 rows and 256 to
+// 160 columns) or rounded to bf16 (256 x 256) in registers, C f32.  With two
+// terms C is bit-identical to the split pass plus launch_gemm_large on the
+// term rows.  gemm_f32a_fits: shapes and alignments it takes;
+// gemm_f32a_supported: and at least 256 tiles of 256 x 256; gemm_f32a_us: the
+// two-term product's predicted time at K = 2048.
+bool gemm_f32a_fits(int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc, const float *a,
+                    const void *w, const void *c);
 bool gemm_f32a_supported(int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
                          const float *a, const void *w, const void *c);
+double gemm_f32a_us(int M, int N);
 bool launch_gemm_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, float *c,
                       int64_t ldc, int M, int N, int K, bool two_terms, hipStream_t st);
 // Three two-term products of the same a in one grid: a . w[i]^T [M][N] to

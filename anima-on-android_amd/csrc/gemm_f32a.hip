@@ -13,9 +13,11 @@
 // product reads back; staging the f32 rows themselves moves the same bytes
 // through L2 as the hi and lo rows would, and the pass and its HBM round trip
 // go away.  Shape of the kernel:
-//   * 256 x 256 tiles of C, 32-element K chunks: a stage is 256 f32 A rows
-//     (128 bytes each) + 256 W rows (64 bytes), 48 KiB; three stages (144
-//     KiB), so a chunk's copies have two chunks' time to land;
+//   * 256 x 256 tiles of C (two terms: or 224, 192 or 160 columns where those
+//     come out more even over the CUs, best_nb below), 32-element K chunks: a
+//     stage is 256 f32 A rows (128 bytes each) + 256 W rows (64 bytes), 48
+//     KiB; three stages (144 KiB), so a chunk's copies have two chunks' time
+//     to land;
 //   * 8 waves as 8 (M) x 1 (N): a wave owns 32 rows of C and all 256
 //     columns (8 accumulators of v_mfma_f32_32x32x16_bf16), so each A row is
 //     read and split by one wave only, and per 16-element K step a wave does
@@ -23,7 +25,7 @@
 //     and 8 W reads; two terms need 24 B/clk of L2 -> LDS at the full MFMA
 //     rate (inside the ~35 B/clk a CU takes), one term 48;
 //   * every wave copies 4 A windows and 2 W windows of each chunk (1 KiB
-//     global_load_lds each); 16-byte pieces are XOR-swizzled (A rows by
+//     global_load_lds each; in narrower tiles some waves 1 W window); 16-byte pieces are XOR-swizzled (A rows by
 //     (row & 7) ^ ((row >> 3) & 1), W rows by (row >> 2) & 3) so each 16-lane
 //     quarter of a fragment read touches 16 distinct bank groups;
 //   * one barrier per chunk, between its two K steps, after every wave has
@@ -65,8 +67,8 @@ constexpr int kFaAEl = kFaBM * kFaBK * 2;        // 16-bit slots of the f32 A pa
 constexpr int kFaWEl = kFaBN * kFaBK;            // 16-bit slots of the W part (16 KiB)
 constexpr int kFaStage = kFaAEl + kFaWEl;        // 48 KiB
 constexpr int kFaACopies = kFaAEl / 512 / kFaWaves;  // 1 KiB windows per wave: 4
-constexpr int kFaWCopies = kFaWEl / 512 / kFaWaves;  // 2
-constexpr int kFaNB = kFaBN / 32;                // accumulator blocks per wave
+constexpr int kFaWCopies = kFaWEl / 512 / kFaWaves;  // most W windows per wave: 2
+constexpr int kFaNB = kFaBN / 32;                // accumulator blocks per wave, widest tile
 
 // The attention operands written in place of C by the fused q/k/v
 // projection (launch_gemm_f32a_qkv): columns [0, HD) are q, [HD, 2HD) k,
@@ -271,9 +273,13 @@ __device__ __forceinline__ void qkv_epilogue(const FaQkv &e, f32x16 (&acc)[kFaNB
     }
 }
 
-template <int TERMS, bool QKV>
+// NB: 32-column blocks of the tile (256 x 32 NB of C).  Narrower tiles than 256
+// columns where they come out more even over the CUs (best_nb below).
+template <int TERMS, bool QKV, int NB>
 __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
 {
+    static_assert(!QKV || NB == kFaNB, "the fused epilogue takes two whole heads");
+    constexpr int BN = 32 * NB;
     __shared__ __attribute__((aligned(16))) u16 smem[kFaStages * kFaStage];
 
     const int tid = threadIdx.x;
@@ -283,15 +289,19 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
 
     const int blk = xcd_major_block();
     const int tn = blk % g.tiles_n, tm = blk / g.tiles_n;
-    const int row0 = tm * kFaBM, col0 = tn * kFaBN;
+    const int row0 = tm * kFaBM, col0 = tn * BN;
 
     // Copies.  A window i of wave w is window 4w + i of the A part (8 rows
     // of 128 bytes): lane l fills slot l & 7 of row (64 win + l) >> 3 with
     // the row's piece slot ^ fa_swz_a(row).  W window i is window 2w + i of
-    // the W part (16 rows of 64 bytes), slot l & 3 of row (64 win + l) >> 2
-    // with piece slot ^ fa_swz_w(row).  Rows past M or N re-read the last
-    // row (their results are not stored).  Byte offsets from the tile's first
-    // row at the chunk's first column.
+    // the W part (16 rows of 64 bytes; 2 NB windows; narrower tiles: w + 8i,
+    // every wave at least one), slot l & 3 of row (64 win + l) >> 2 with piece
+    // slot ^ fa_swz_w(row).  Rows past M or N re-read the last row (their
+    // results are not stored).  Byte offsets from the tile's first row at the
+    // chunk's first column.
+    const auto wwin = [&](int i) {
+        return NB == kFaNB ? wave * kFaWCopies + i : wave + kFaWaves * i;
+    };
     unsigned aoff[kFaACopies], woff[kFaWCopies];
 #pragma unroll
     for (int i = 0; i < kFaACopies; ++i) {
@@ -302,7 +312,7 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
     }
 #pragma unroll
     for (int i = 0; i < kFaWCopies; ++i) {
-        const int f = (wave * kFaWCopies + i) * 64 + lane;
+        const int f = wwin(i) * 64 + lane;
         const int r = f >> 2, pc = (f & 3) ^ fa_swz_w(r);
         const int rr = min(col0 + r, g.N - 1) - col0;
         woff[i] = unsigned(int64_t(rr) * g.ldw * 2 + 16 * pc);
@@ -319,12 +329,30 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
             dma16s(asrc + int64_t(c) * kFaBK * 4, aoff[i], st + (wave * kFaACopies + i) * 512);
         else
             dma16s(wsrc + int64_t(c) * kFaBK * 2, woff[i - kFaACopies],
-                   st + kFaAEl + (wave * kFaWCopies + i - kFaACopies) * 512);
+                   st + kFaAEl + wwin(i - kFaACopies) * 512);
     };
+    // Copies of this wave per chunk: its second W window may be past the tile.
+    constexpr int kCopies = kFaACopies + kFaWCopies;
+    const bool all = NB == kFaNB || wave + kFaWaves < 2 * NB;
     auto dma = [&](int c, int stage) {
 #pragma unroll
-        for (int i = 0; i < kFaACopies + kFaWCopies; ++i)
+        for (int i = 0; i < kCopies - 1; ++i)
             dma_one(c, stage, i);
+        if (all)
+            dma_one(c, stage, kCopies - 1);
+    };
+    // Until at most n later chunks' copies are in flight.
+    auto wait1 = [&] {
+        if (all)
+            wait_vmcnt<kCopies>();
+        else
+            wait_vmcnt<kCopies - 1>();
+    };
+    auto wait2 = [&] {
+        if (all)
+            wait_vmcnt<2 * kCopies>();
+        else
+            wait_vmcnt<2 * (kCopies - 1)>();
     };
 
     // Fragments of K step t (elements 16t .. 16t + 15 of the chunk): this
@@ -332,12 +360,12 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
     // 16-byte pieces of f32) and of W rows 32 nb + col (one piece of bf16).
     const int arow = wave * 32 + col;
     const int aswz = fa_swz_a(arow);
-    auto frags = [&](const u16 *st, int t, bf16x8 (&af)[2], bf16x8 (&wf)[kFaNB]) {
+    auto frags = [&](const u16 *st, int t, bf16x8 (&af)[2], bf16x8 (&wf)[NB]) {
         const int p0 = 2 * (2 * t + half);
         const f32x4 x0 = *reinterpret_cast<const f32x4 *>(st + arow * 64 + 8 * (p0 ^ aswz));
         const f32x4 x1 = *reinterpret_cast<const f32x4 *>(st + arow * 64 + 8 * ((p0 + 1) ^ aswz));
 #pragma unroll
-        for (int nb = 0; nb < kFaNB; ++nb) {
+        for (int nb = 0; nb < NB; ++nb) {
             const int r = 32 * nb + col;
             wf[nb] = *reinterpret_cast<const bf16x8 *>(st + kFaAEl + r * kFaBK +
                                                        8 * ((2 * t + half) ^ fa_swz_w(r)));
@@ -350,15 +378,15 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
             af[1] = __builtin_bit_cast(bf16x8, uint4{l0.x, l0.y, l1.x, l1.y});
     };
 
-    f32x16 acc[kFaNB];
+    f32x16 acc[NB];
 #pragma unroll
-    for (int nb = 0; nb < kFaNB; ++nb)
+    for (int nb = 0; nb < NB; ++nb)
         acc[nb] = f32x16{};
-    bf16x8 af[2][2], wf[2][kFaNB];
+    bf16x8 af[2][2], wf[2][NB];
     // Per accumulator the hi product, then the lo product.
     auto mfmas = [&](int set) {
 #pragma unroll
-        for (int nb = 0; nb < kFaNB; ++nb) {
+        for (int nb = 0; nb < NB; ++nb) {
             acc[nb] = mfma_bf16(af[set][0], wf[set][nb], acc[nb]);
             if (TERMS == 2)
                 acc[nb] = mfma_bf16(af[set][1], wf[set][nb], acc[nb]);
@@ -366,7 +394,6 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
     };
 
     const int total = g.chunks;
-    constexpr int kCopies = kFaACopies + kFaWCopies;  // per wave and chunk
     dma(0, 0);
     if (total > 1)
         dma(1, 1);
@@ -374,9 +401,9 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
         dma(2, 2);
     // Chunk 0's copies landed: the later chunks' may still be in flight.
     if (total > 2)
-        wait_vmcnt<2 * kCopies>();
+        wait2();
     else if (total > 1)
-        wait_vmcnt<kCopies>();
+        wait1();
     else
         wait_vmcnt<0>();
     ring_barrier();
@@ -393,7 +420,7 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
             // step-1 fragments above; the barrier waits for those reads), so
             // chunk c's stage takes chunk c + 3 while the step-1 MFMAs run.
             if (c + 2 < total)
-                wait_vmcnt<kCopies>();
+                wait1();
             else
                 wait_vmcnt<0>();
             ring_barrier();
@@ -404,20 +431,22 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
         // the MFMAs.
         const bool copies = c + 3 < total;
 #pragma unroll
-        for (int nb = 0; nb < kFaNB; ++nb) {
+        for (int nb = 0; nb < NB; ++nb) {
             acc[nb] = mfma_bf16(af[1][0], wf[1][nb], acc[nb]);
             if (TERMS == 2)
                 acc[nb] = mfma_bf16(af[1][1], wf[1][nb], acc[nb]);
             __builtin_amdgcn_sched_barrier(0);
-            if (copies && nb < kCopies)
+            if (copies && nb < kCopies - 1)
                 dma_one(c + 3, c % kFaStages, nb);
+            if (copies && all && nb == (NB < kCopies ? NB : kCopies) - 1)
+                dma_one(c + 3, c % kFaStages, kCopies - 1);
             __builtin_amdgcn_sched_barrier(0);
         }
         if (more)
             frags(smem + ((c + 1) % kFaStages) * kFaStage, 0, af[0], wf[0]);
     }
 
-    if (QKV) {
+    if constexpr (QKV) {
         qkv_epilogue(g.qkv, acc, reinterpret_cast<float *>(smem), g.M, row0, col0, wave, lane);
         return;
     }
@@ -428,9 +457,9 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
     // round of tiles then overlap the next round's loads better (8192 x 8192
     // x 2048: 0.498 -> 0.480 ms, 8192 x 2048 x 2048 0.1203 -> 0.1188 ms on one
     // box).
-    const bool full = row0 + kFaBM <= g.M && col0 + kFaBN <= g.N;
+    const bool full = row0 + kFaBM <= g.M && col0 + BN <= g.N;
 #pragma unroll
-    for (int nb = 0; nb < kFaNB; ++nb) {
+    for (int nb = 0; nb < NB; ++nb) {
         const int n = col0 + 32 * nb + col;
         float *c = g.c + part * g.c_step + pcol0 + 32 * nb + col;
 #pragma unroll
@@ -445,28 +474,65 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
 
 }  // namespace
 
+namespace {
+// Predicted time (us at K = 2048) of the two-term product in 256 x 32 nb tiles on
+// 256 CUs, fitted to 23 shapes of 1100 to 8192 rows on MI355X (within 6 %): a
+// full round is bound by power; one that fills part of the CUs clocks higher
+// until a tile's own copies and latencies bound it.
+double tiles_us(int64_t tiles_m, int64_t N, int nb)
+{
+    const int64_t tiles = tiles_m * ((N + 32 * nb - 1) / (32 * nb));
+    const int64_t rest = tiles % 256;
+    return double(tiles / 256) * (30.0 + 10.5 * nb) +
+           (rest ? std::max(24.0 + 7.25 * nb, 30.0 + 0.041 * double(rest * nb)) : 0.0);
+}
+
+// The tile width (32-column blocks, 5 to 8) that comes out best: 4608 x 2048 x 8192
+// runs 144 tiles of 256 columns in 305 us, 234 of 160 in 289; 3072 x 6144 x 2048
+// 288 in 191, 468 in 153; 2048 x 6144 x 2048 192 in 100, 256 of 192 in 94.
+int best_nb(int M, int N)
+{
+    const int64_t tm = (int64_t(M) + kFaBM - 1) / kFaBM;
+    int best = kFaNB;
+    for (int nb = 5; nb < kFaNB; ++nb)
+        if (tiles_us(tm, N, nb) < 0.98 * tiles_us(tm, N, best))
+            best = nb;
+    return best;
+}
+}  // namespace
+
+double gemm_f32a_us(int M, int N)
+{
+    return tiles_us((int64_t(M) + kFaBM - 1) / kFaBM, N, best_nb(M, N));
+}
+
 // Shapes the kernel takes: K a multiple of 32, 16-byte aligned A and W rows,
-// byte offsets of a tile's rows within 32 bits, and at least one full round
-// of workgroups (256 tiles of 256 x 256).
-bool gemm_f32a_supported(int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
-                         const float *a, const void *w, const void *c)
+// byte offsets of a tile's rows within 32 bits.
+bool gemm_f32a_fits(int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc, const float *a,
+                    const void *w, const void *c)
 {
     const auto al = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    if (M <= 0 || N <= 0 || K <= 0 || K % kFaBK)
-        return false;
-    const int64_t tiles = int64_t((M + kFaBM - 1) / kFaBM) * ((N + kFaBN - 1) / kFaBN);
-    return tiles >= 256 && tiles < (int64_t(1) << 31) && lda >= K && ldw >= K && ldc >= N &&
+    return M > 0 && N > 0 && K > 0 && K % kFaBK == 0 && lda >= K && ldw >= K && ldc >= N &&
            lda % 4 == 0 && ldw % 8 == 0 && al(a) && al(w) &&
            (reinterpret_cast<uintptr_t>(c) & 3) == 0 &&
            int64_t(kFaBM) * lda * 4 < (int64_t(1) << 31) &&
            int64_t(kFaBN) * ldw * 2 < (int64_t(1) << 31);
 }
 
+// And at least one full round of workgroups (256 tiles of 256 x 256).
+bool gemm_f32a_supported(int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
+                         const float *a, const void *w, const void *c)
+{
+    const int64_t tiles = ((int64_t(M) + kFaBM - 1) / kFaBM) * ((int64_t(N) + kFaBN - 1) / kFaBN);
+    return tiles >= 256 && tiles < (int64_t(1) << 31) &&
+           gemm_f32a_fits(M, N, K, lda, ldw, ldc, a, w, c);
+}
+
 namespace {
-// One part of N columns, or three of part_n.
+// One part of N columns, or three of part_n, in tiles of 32 nb columns.
 bool launch_parts(const float *a, int64_t lda, const uint16_t *const *w, int parts, int64_t ldw,
                   float *c, int64_t c_step, int64_t ldc, int M, int part_n, int K, bool two_terms,
-                  hipStream_t st)
+                  int nb, hipStream_t st)
 {
     FaArgs g{};
     g.a = a;
@@ -480,13 +546,17 @@ bool launch_parts(const float *a, int64_t lda, const uint16_t *const *w, int par
     g.M = M;
     g.N = parts * part_n;
     g.part_n = part_n;
-    g.tiles_n = (g.N + kFaBN - 1) / kFaBN;
+    g.tiles_n = (g.N + 32 * nb - 1) / (32 * nb);
     g.chunks = K / kFaBK;
-    const dim3 grid(unsigned(((M + kFaBM - 1) / kFaBM) * g.tiles_n)), block(kFaWaves * 64);
-    if (two_terms)
-        hipLaunchKernelGGL((gemm_f32a_kernel<2, false>), grid, block, 0, st, g);
-    else
-        hipLaunchKernelGGL((gemm_f32a_kernel<1, false>), grid, block, 0, st, g);
+    const int64_t tiles = int64_t((M + kFaBM - 1) / kFaBM) * g.tiles_n;
+    if (tiles > INT32_MAX)
+        return fail("gemm_f32a: problem too large for one launch");
+    const auto kernel = !two_terms ? gemm_f32a_kernel<1, false, 8>
+                        : nb == 5  ? gemm_f32a_kernel<2, false, 5>
+                        : nb == 6  ? gemm_f32a_kernel<2, false, 6>
+                        : nb == 7  ? gemm_f32a_kernel<2, false, 7>
+                                   : gemm_f32a_kernel<2, false, 8>;
+    hipLaunchKernelGGL(kernel, dim3(unsigned(tiles)), dim3(kFaWaves * 64), 0, st, g);
     return hip_ok(hipGetLastError(), "gemm_f32a_kernel launch");
 }
 }  // namespace
@@ -494,9 +564,11 @@ bool launch_parts(const float *a, int64_t lda, const uint16_t *const *w, int par
 bool launch_gemm_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, float *c,
                       int64_t ldc, int M, int N, int K, bool two_terms, hipStream_t st)
 {
-    if (!gemm_f32a_supported(M, N, K, lda, ldw, ldc, a, w, c))
+    if (!gemm_f32a_fits(M, N, K, lda, ldw, ldc, a, w, c))
         return fail("gemm_f32a: unsupported shape or alignment");
-    return launch_parts(a, lda, &w, 1, ldw, c, 0, ldc, M, N, K, two_terms, st);
+    // One term is bound by its copies, which narrower tiles repeat.
+    return launch_parts(a, lda, &w, 1, ldw, c, 0, ldc, M, N, K, two_terms,
+                        two_terms ? best_nb(M, N) : kFaNB, st);
 }
 
 bool gemm_f32a_three_supported(int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
@@ -512,7 +584,7 @@ bool launch_gemm_f32a_three(const float *a, int64_t lda, const uint16_t *const w
 {
     if (!gemm_f32a_three_supported(M, N, K, lda, ldw, ldc, a, w, c))
         return fail("gemm_f32a: unsupported shape or alignment (three products)");
-    return launch_parts(a, lda, w, 3, ldw, c, c_step, ldc, M, N, K, true, st);
+    return launch_parts(a, lda, w, 3, ldw, c, c_step, ldc, M, N, K, true, kFaNB, st);
 }
 
 bool gemm_f32a_qkv_supported(const float *a, int64_t lda, const uint16_t *const w[3], int64_t ldw,
@@ -525,8 +597,8 @@ bool gemm_f32a_qkv_supported(const float *a, int64_t lda, const uint16_t *const 
     const int64_t M = int64_t(p.B) * p.S, HD = int64_t(p.H) * 128;
     if (M > INT32_MAX || 3 * HD > INT32_MAX)
         return false;
-    return al(w[1]) && al(w[2]) && p.qo && p.ko && p.vo && al(p.qo) && al(p.ko) && al(p.vo) && (!p.w[0] || al(p.w[0])) &&
-           (!p.w[1] || al(p.w[1])) && (!p.freqs || al(p.freqs)) &&
+    return al(w[1]) && al(w[2]) && p.qo && p.ko && p.vo && al(p.qo) && al(p.ko) && al(p.vo) &&
+           (!p.w[0] || al(p.w[0])) && (!p.w[1] || al(p.w[1])) && (!p.freqs || al(p.freqs)) &&
            gemm_f32a_supported(int(M), int(3 * HD), K, lda, ldw, 3 * HD, a, w[0], p.qo);
 }
 
@@ -561,7 +633,7 @@ bool launch_gemm_f32a_qkv(const float *a, int64_t lda, const uint16_t *const w[3
     g.qkv.eps = p.eps;
     g.qkv.terms = p.mode == kAttnF32X3 ? 1 : 0;
     const dim3 grid(unsigned(((g.M + kFaBM - 1) / kFaBM) * g.tiles_n)), block(kFaWaves * 64);
-    hipLaunchKernelGGL((gemm_f32a_kernel<2, true>), grid, block, 0, st, g);
+    hipLaunchKernelGGL((gemm_f32a_kernel<2, true, kFaNB>), grid, block, 0, st, g);
     return hip_ok(hipGetLastError(), "gemm_f32a_kernel (q/k/v) launch");
 }
 

@@ -23,6 +23,7 @@
 
 #include <hipblaslt/hipblaslt.h>
 
+#include <algorithm>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -307,6 +308,29 @@ size_t linear_scratch_bytes(int M, int K, bool exact)
            (small_m_path(M, K, exact) ? kGemmBf16MaxWorkspace : 0);
 }
 
+// Always where 256 x 256 tiles fill the GPU.  Below that, past the small-M
+// kernel's rows, where its prediction beats those of the other ways by 4 % (at
+// K = 2048, us, fitted to the same shapes): the 128 x 256 kernel where its
+// tiles fill the GPU (62 a round, a last round of at least 40: 4096 x 2048 62
+// against 72 here, 4608 x 2048 102 against 75), or the split pass and two
+// library products (16 plus 0.9 PFLOP/s: 2048 x 2048 54 against 60, 3584 x
+// 2048 76 against 67, 1536 x 6144 103 against 76).
+bool linear_takes_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, const float *c,
+                       int64_t ldc, int M, int N, int K)
+{
+    if (gemm_f32a_supported(M, N, K, lda, ldw, ldc, a, w, c))
+        return true;
+    if (!gemm_f32a_fits(M, N, K, lda, ldw, ldc, a, w, c) || small_m_path(M, K, true))
+        return false;
+    double other = 16.0 + 4.0 * M * double(N) * 2048 / 0.9e9;
+    if (gemm_large_f32a_supported(M, N, K, lda, ldw, ldc, a, w, c)) {
+        const int64_t tiles = ((int64_t(M) + 127) / 128) * ((int64_t(N) + 255) / 256);
+        const int64_t rest = tiles % 256;
+        other = double(tiles / 256) * 62.0 + (rest ? std::max(40.0, 0.24 * double(rest)) : 0.0);
+    }
+    return 1.04 * gemm_f32a_us(M, N) <= other;
+}
+
 bool launch_linear(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, float *c,
                    int64_t ldc, int M, int N, int K, bool exact, void *scratch,
                    size_t scratch_bytes, hipStream_t st)
@@ -329,11 +353,10 @@ bool launch_linear(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, 
     if (!scratch || scratch_bytes < linear_scratch_bytes(M, K, exact) ||
         (reinterpret_cast<uintptr_t>(scratch) & 15u) != 0)
         return fail("linear: scratch smaller than linear_scratch_bytes() or not 16-byte aligned");
-    // Large M, f32 modes: the kernel splits f32 A into its hi and lo terms in
+    // Large M, f32 modes: the kernels split f32 A into its hi and lo terms in
     // registers, so the terms make no round trip through HBM; bit-identical to
-    // the split + two-term product below.  256 x 256 tiles where they fill the
-    // GPU, else 128 x 256.
-    if (exact && gemm_f32a_supported(M, N, K, lda, ldw, ldc, a, w, c))
+    // the split + two-term product of gemm_large.hip below.
+    if (exact && linear_takes_f32a(a, lda, w, ldw, c, ldc, M, N, K))
         return launch_gemm_f32a(a, lda, w, ldw, c, ldc, M, N, K, true, st);
     // One term (bf16 mode): the same kernel rounding A to bf16 in registers
     // beats the split pass + library product where N and K are at most 2048
