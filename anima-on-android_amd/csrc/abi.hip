@@ -735,10 +735,15 @@ bool sdpa_heads(Runtime &r, int64_t h0, int nh, int S_q, int S_kv, int D, float 
     return x3 ? launch_flash_x3(p, st, scr) : launch_flash_bf16(p, st, scr);
 }
 
-// Head groups of a host-pointer SDPA: the most groups (4 or 2) that still
-// fill the GPU each
-// when the copies are large, else one.  Group g+1 uploads while group g
-// computes, and group g's output comes back while later groups upload.
+// Head groups of a host-pointer SDPA: when the copies are large, the most
+// groups (4 or 2) that still fill the GPU each, or two where the whole call does
+// not fill it either (its kernels share out the keys of each query tile, and
+// the groups' do the same); else one.  Group g+1 uploads while group g computes,
+// and group g's output comes back while later groups upload.  In that last
+// case two groups against one ran 1.91 against 2.32 ms (BH = 32, S = 1024), 1.97
+// against 2.42 (16, 2048) and 2.12 against 2.79 (8, 4096); four 2.30, 2.28 and
+// 2.54, each group's copies paying their own latencies; at 50 MB of copies two
+// were 2 % faster, at 34 MB 8 to 12 % slower.
 int sdpa_groups(int BH, int S_q, int S_kv, int D)
 {
     const int64_t bytes = int64_t(BH) * (2 * int64_t(S_q) + 2 * int64_t(S_kv)) * D * 4;
@@ -750,7 +755,7 @@ int sdpa_groups(int BH, int S_q, int S_kv, int D)
         if (flash_fills_gpu(BH / G, S_q, D))
             return G;
     }
-    return 1;
+    return !flash_fills_gpu(BH, S_q, D) && BH % 2 == 0 ? 2 : 1;
 }
 
 // Shared body of the host-pointer SDPA entries ([BH, S, D] f32 host arrays).

@@ -135,3 +135,20 @@ def test_attention_four_batch_groups_equal_the_single_batch_calls():
     err = float(np.abs(full[3, :, 9] - ref).max())
     print(f"pipeline attention four groups b=3 h=9: max-abs {err:.3e}", flush=True)
     assert err <= 1e-4
+
+
+@pytest.mark.parametrize("mode", [rt.F32, rt.F32X3, rt.BF16])
+@pytest.mark.parametrize("BH,Sq,Sk", [(32, 1024, 1024), (6, 2001, 9003)])
+def test_two_groups_of_a_grid_that_does_not_fill_the_gpu(BH, Sq, Sk, mode):
+    """64 MiB of copies or more and fewer query tiles than CUs: two groups, each
+    like a call on half of the slices alone."""
+    rng = np.random.default_rng(BH + Sq + mode)
+    q = rng.standard_normal((BH, Sq, 128), dtype=np.float32)
+    k, v = (rng.standard_normal((BH, Sk, 128), dtype=np.float32) for _ in range(2))
+    print(f"pipeline case BH={BH} Sq={Sq} Sk={Sk} mode={mode}", flush=True)
+    full = rt.sdpa(q, k, v, mode=mode)
+    h = BH // 2
+    halves = np.concatenate([rt.sdpa(q[:h], k[:h], v[:h], mode=mode),
+                             rt.sdpa(q[h:], k[h:], v[h:], mode=mode)])
+    np.testing.assert_array_equal(full, halves)
+    _check_slices(full, q, k, v, (0, BH - 1), mode, "small grid groups")
