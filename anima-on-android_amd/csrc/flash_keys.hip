@@ -18,10 +18,13 @@
 // bound by the L2 -> LDS stream (128 KiB per round of four tiles, about 35 bytes
 // per clock and CU) where the grid fills the GPU.
 // Whole attention calls on MI355X before and now, 16 heads (f32x3 / bf16): self
-// 256 tokens 24.7 -> 22.5 / 17.8 -> 16.4 us, 1024 tokens 50.4 -> 46.6 / 39.1 ->
-// 30.8; cached cross-attention, query rows normalised in here, 256 x 512
-// 28.8 -> 23.1 / 20.7 -> 16.8, 1024 x 512 34.5 -> 24.6 / 22.6 -> 17.9.  A round
-// takes about 4 us (f32x3): each of its two phases waits for 64 KiB of copies.
+// 256 tokens 24.7 -> 22.3 / 17.8 -> 15.5 us, 1024 tokens 50.4 -> 45.6 / 39.1 ->
+// 30.3; cached cross-attention, query rows normalised in here, 2 x 256 on 512
+// 28.8 -> 17.9 / 20.7 -> 12.0, 1024 x 512 34.5 -> 20.0 / 22.6 -> 12.7.  Cycles of
+// 2 x 256 tokens, self f32x3 (31.6k): 11.4k until the first K tiles and Q are
+// there, 2.1k to 2.4k a phase of MFMAs and 0.6k to 0.9k more for its copies
+// (waiting for K and V^T with a barrier of its own each, so that more copies are
+// in flight, was 3 to 16 % slower), 6.2k for the merge.
 //
 // Per key group one K tile and one V^T tile (16 KiB each: 32 keys of terms, 64
 // of bf16), single-buffered and refilled in turn: V^T lands while the scores
@@ -60,6 +63,75 @@ struct KeysArgs {
 // bits: this file is compiled without NaN comparisons).
 __device__ __forceinline__ bool joins(const float2 &p) { return (__float_as_uint(p.y) << 1) != 0; }
 
+// The terms of the workgroup's 64 raw rows, bit for bit those of the row prologue
+// (prologue.hip) and q_terms_from_raw: one lane per row adds the squares in
+// index order, every thread then scales, rotates and splits its own four
+// float4 (row tid / 32 + 16 i, columns 4 (tid % 32)), and the waves read their
+// fragments back.  q_terms_from_raw in every wave did the work of a row four
+// times over in some 1500 instructions run once, most of their time spent
+// fetching them: 18.7k of the 52k cycles of 256 x 512 f32x3, KQT here.
+template <int TERMS>
+__device__ __forceinline__ void keys_q_terms(const KeysArgs &a, float *rows, const f32x4 (&v)[4],
+                                             int q0, int tid, bf16x8 (&qh)[8], bf16x8 (&ql)[8])
+{
+#pragma clang fp contract(off)
+    constexpr int kTermPitch = TERMS * kD + 8;  // 16-bit elements, 16 bytes against conflicts
+    __shared__ float inv[kRowsPerBlock];
+    if (tid < kRowsPerBlock) {
+        const float *row = rows + tid * kPitch;
+        float ss = 0.0f;
+#pragma unroll 4
+        for (int j = 0; j < kD / 4; ++j) {
+            const f32x4 x = *reinterpret_cast<const f32x4 *>(row + 4 * j);
+            ss = ss + x.x * x.x;
+            ss = ss + x.y * x.y;
+            ss = ss + x.z * x.z;
+            ss = ss + x.w * x.w;
+        }
+        inv[tid] = inv_rms(ss, kD, a.eps);
+    }
+    const int c4 = tid & 31, p0 = 4 * (c4 & 15);
+    f32x4 w = f32x4{1.f, 1.f, 1.f, 1.f};
+    if (a.qw)
+        w = *reinterpret_cast<const f32x4 *>(a.qw + 4 * c4);
+    __syncthreads();  // the sums are there, the rows are read
+    u16 *const terms = reinterpret_cast<u16 *>(rows);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int r = (tid >> 5) + 16 * i;
+        f32x4 y = v[i] * inv[r];
+        if (a.qw)
+            y = y * w;
+        if (a.qf) {
+            // Pairs (p, p + 64): the other half's values are 16 lanes away.
+            const bool hi = c4 >= 16;
+            const float *fq =
+                a.qf + int64_t(min(q0 + r, a.S_q - 1)) * (2 * kD) + 4 * p0 + (hi ? 2 : 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float2 c = *reinterpret_cast<const float2 *>(fq + 4 * e);
+                const float other = __shfl_xor(y[e], 16);
+                const float ya = hi ? other : y[e], yb = hi ? y[e] : other;
+                y[e] = c.x * ya + c.y * yb;
+            }
+        }
+        uint2 th, tl;
+        split_terms4(y, th, tl);
+        *reinterpret_cast<uint2 *>(terms + r * kTermPitch + 4 * c4) = th;
+        if (TERMS == 2)
+            *reinterpret_cast<uint2 *>(terms + r * kTermPitch + kD + 4 * c4) = tl;
+    }
+    __syncthreads();
+    const int lane = tid & 63, row = 32 * ((tid >> 6) & 1) + (lane & 31);
+    const u16 *src = terms + row * kTermPitch + 64 * (lane >> 5);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+        qh[t] = *reinterpret_cast<const bf16x8 *>(src + 8 * t);
+        if (TERMS == 2)
+            ql[t] = *reinterpret_cast<const bf16x8 *>(src + kD + 8 * t);
+    }
+}
+
 template <int TERMS>
 __global__ __launch_bounds__(512, 1) void flash_keys_d128(KeysArgs a)
 {
@@ -73,6 +145,7 @@ __global__ __launch_bounds__(512, 1) void flash_keys_d128(KeysArgs a)
     __shared__ __attribute__((aligned(16))) unsigned char
         smem[kMergeBytes > kRingBytes ? kMergeBytes : kRingBytes];
     __shared__ float2 ml[8][32];  // (max, sum) per wave and row
+    __shared__ float sums[8][32];  // sums against the row's max
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -188,10 +261,7 @@ __global__ __launch_bounds__(512, 1) void flash_keys_d128(KeysArgs a)
             *reinterpret_cast<f32x4 *>(rows + (f >> 5) * kPitch + 4 * (f & 31)) = v[i];
         }
         __syncthreads();
-        q_terms_from_raw<TERMS == 2>(rows + (32 * rg + col) * kPitch, a.qw,
-                                     a.qf ? a.qf + int64_t(min(qrow, a.S_q - 1)) * 4 * kD / 2
-                                          : nullptr,
-                                     a.eps, true, half, qh, ql);
+        keys_q_terms<TERMS>(a, rows, v, q0, tid, qh, ql);
     } else {
         const u16 *qr = a.q + b * a.qb + h * a.qh + int64_t(min(qrow, a.S_q - 1)) * a.qs;
         const bf16x8 *src = reinterpret_cast<const bf16x8 *>(qr + 64 * half);
@@ -317,6 +387,8 @@ __global__ __launch_bounds__(512, 1) void flash_keys_d128(KeysArgs a)
             mx = fmaxf(mx, p.x);
     }
     const float w = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
+    if (half == 0)
+        sums[wave][col] = m == -INFINITY ? 0.0f : l * w;
     float *const part = reinterpret_cast<float *>(smem);
 #pragma unroll
     for (int d = 0; d < 4; ++d)
@@ -329,29 +401,19 @@ __global__ __launch_bounds__(512, 1) void flash_keys_d128(KeysArgs a)
                                        acc_row(4 * g, half)) = v;
         }
     __syncthreads();
-#pragma unroll
+#pragma unroll 1
     for (int i = 0; i < kRowsPerBlock * 32 / 512; ++i) {
         const int f = tid + 512 * i, r = f >> 5, c4 = f & 31;
         if (q0 + r >= a.S_q)
             continue;
         const int r0 = r >> 5, rr = r & 31;
-        float top = -INFINITY;
-#pragma unroll
-        for (int g = 0; g < kGroups; ++g) {
-            const float2 p = ml[2 * g + r0][rr];
-            if (joins(p))
-                top = fmaxf(top, p.x);
-        }
         float sum = 0.0f;
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int g = 0; g < kGroups; ++g) {
-            const float2 p = ml[2 * g + r0][rr];
-            if (joins(p)) {
-                sum += p.y * __builtin_amdgcn_exp2f(p.x - top);
-                v += *reinterpret_cast<const f32x4 *>(part + ((2 * g + r0) * 32 + rr) * kPitch +
-                                                      4 * c4);
-            }
+            sum += sums[2 * g + r0][rr];
+            v += *reinterpret_cast<const f32x4 *>(part + ((2 * g + r0) * 32 + rr) * kPitch +
+                                                  4 * c4);
         }
         v *= sum > 0.0f ? 1.0f / sum : 0.0f;  // a NaN sum has NaN in v
         const int q = q0 + r;
