@@ -132,6 +132,8 @@ __global__ __launch_bounds__(256) void rows_kernel(RowArgs a)
         if (a.norm) {
             const float *row = xs + rr * pitch;
             float ss = 0.0f;
+            // 16 elements' reads ahead of their adds (two rows of 2048: 34 -> 28 us).
+#pragma unroll 16
             for (int d = 0; d < D; ++d)
                 ss = ss + row[d] * row[d];
             f = inv_rms(ss, D, a.eps);
