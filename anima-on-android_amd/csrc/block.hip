@@ -477,9 +477,9 @@ bool run_attention_block(const BlockProblem &p, void *scratch, size_t scratch_by
     // library GEMM does not take (launch_linear's exact f32 fallback needs
     // O itself), or one that the f32-activation kernel runs better than the
     // kernels on terms (4608 rows: 75 against 96 us): f32 O at o.
+    const bool lib = linear_terms_supported(int(M), Dm, HD, p.wo, HD, y, Dm);
     const bool f32a_out = !bf16 && linear_takes_f32a(o, HD, p.wo, HD, y, Dm, int(M), Dm, HD);
-    const bool terms_out = D == 128 && !f32a_out &&
-                           linear_terms_supported(int(M), Dm, HD, p.wo, HD, y, Dm);
+    const bool terms_out = D == 128 && !f32a_out && lib;
     const int64_t kp = linear_terms_ld(HD);
     const size_t hi_bytes = round_up256(size_t(M) * size_t(kp) * 2);
     uint16_t *ohi = static_cast<uint16_t *>(lin);
@@ -496,16 +496,20 @@ bool run_attention_block(const BlockProblem &p, void *scratch, size_t scratch_by
 
     // output_proj (numpy_dit.py:294-296) and the gated residual.  bf16 mode:
     // one GEMM per batch entry whose per-channel scale is the gate and whose
-    // C and D are the residual stream.  f32 mode (two terms, each pass would
-    // read and write the residual again), or a shape the library GEMM does
-    // not take with a per-channel scale: the projection into y, then a
-    // residual pass.
+    // C and D are the residual stream.  f32 modes where the f32-activation
+    // kernel runs the product: its epilogue updates the residual.  Otherwise
+    // (two library passes would read and write the residual twice), or for a
+    // shape the library GEMM does not take with a per-channel scale: the
+    // projection into y, then a residual pass.
     if (bf16 && linear_residual_supported(S, Dm, HD, p.wo, HD, p.x, Dm))
         return terms_out
                    ? launch_linear_residual_terms(ohi, p.wo, HD, p.x, Dm, p.mod + 2 * int64_t(Dm),
                                                   3 * int64_t(Dm), B, S, Dm, HD, st)
                    : launch_linear_residual(o, HD, p.wo, HD, p.x, Dm, p.mod + 2 * int64_t(Dm),
                                             3 * int64_t(Dm), B, S, Dm, HD, lin, s.lin, st);
+    if (f32a_out && lib && S >= 32)
+        return launch_gemm_f32a_residual(o, HD, p.wo, HD, p.x, Dm, p.mod + 2 * int64_t(Dm),
+                                         3 * int64_t(Dm), S, int(M), Dm, HD, st);
     const size_t terms_bytes = hi_bytes * (bf16 ? 1 : 2);
     const bool ok =
         terms_out ? launch_linear_terms(ohi, olo, p.wo, HD, y, Dm, int(M), Dm, HD, st,

@@ -268,6 +268,11 @@ bool gemm_f32a_supported(int M, int N, int K, int64_t lda, int64_t ldw, int64_t 
 double gemm_f32a_us(int M, int N);
 bool launch_gemm_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, float *c,
                       int64_t ldc, int M, int N, int K, bool two_terms, hipStream_t st);
+// x [M][ldx] += gate[m / S] * (a W^T), the two-term product as launch_gemm_f32a's
+// (gate rows of N gate_stride apart; S >= 32 divides M).
+bool launch_gemm_f32a_residual(const float *a, int64_t lda, const uint16_t *w, int64_t ldw,
+                               float *x, int64_t ldx, const float *gate, int64_t gate_stride,
+                               int S, int M, int N, int K, hipStream_t st);
 // Three two-term products of the same a in one grid: a . w[i]^T [M][N] to
 // c + i * c_step, each bit-identical to launch_gemm_f32a's; N a multiple of
 // 256, and a grid of at least 256 tiles over all three.

@@ -93,6 +93,10 @@ struct FaArgs {
     int64_t lda, ldw, ldc, c_step;
     int M, N, part_n, tiles_n, chunks;
     FaQkv qkv;        // QKV kernels only
+    // Residual kernels only: c is the residual x, c[m][n] += gate[m / S][n] * C.
+    const float *gate;  // rows gate_stride apart
+    int64_t gate_stride;
+    int S;              // at least 32
 };
 
 constexpr int kQkvPitch = 132;  // floats per staged row of a head block (128 + 4 against conflicts)
@@ -275,7 +279,8 @@ __device__ __forceinline__ void qkv_epilogue(const FaQkv &e, f32x16 (&acc)[kFaNB
 
 // NB: 32-column blocks of the tile (256 x 32 NB of C).  Narrower tiles than 256
 // columns where they come out more even over the CUs (best_nb below).
-template <int TERMS, bool QKV, int NB>
+// RES: the gated residual update in place of C.
+template <int TERMS, bool QKV, int NB, bool RES = false>
 __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
 {
     static_assert(!QKV || NB == kFaNB, "the fused epilogue takes two whole heads");
@@ -450,6 +455,30 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
         qkv_epilogue(g.qkv, acc, reinterpret_cast<float *>(smem), g.M, row0, col0, wave, lane);
         return;
     }
+    if constexpr (RES) {
+        // The wave's 32 rows meet at most one batch boundary (S >= 32).
+        const int mw = row0 + wave * 32;
+        const int b0 = mw / g.S, bnd = (b0 + 1) * g.S;
+        const int b1 = min(b0 + 1, (g.M - 1) / g.S);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            const int n = col0 + 32 * nb + col, nr = min(n, g.N - 1);
+            const float g0 = g.gate[int64_t(min(b0, b1)) * g.gate_stride + nr];
+            const float g1 = g.gate[int64_t(b1) * g.gate_stride + nr];
+            float x[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                x[r] = g.c[int64_t(min(mw + acc_row(r, half), g.M - 1)) * g.ldc + nr];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = mw + acc_row(r, half);
+                if (m < g.M && n < g.N)
+                    g.c[int64_t(m) * g.ldc + n] = x[r] + (m < bnd ? g0 : g1) * acc[nb][r];
+            }
+        }
+        return;
+    }
+
     // Lane (col, half) of accumulator nb holds C[m][n] for n = col0 + 32 nb +
     // col and m = row0 + wave * 32 + acc_row(r, half): for one register, 32
     // lanes cover 128 consecutive bytes of a row.  Nontemporal (streaming)
@@ -529,10 +558,12 @@ bool gemm_f32a_supported(int M, int N, int K, int64_t lda, int64_t ldw, int64_t 
 }
 
 namespace {
-// One part of N columns, or three of part_n, in tiles of 32 nb columns.
+// One part of N columns, or three of part_n, in tiles of 32 nb columns; with a
+// gate, the gated residual update of c (two terms, one part).
 bool launch_parts(const float *a, int64_t lda, const uint16_t *const *w, int parts, int64_t ldw,
                   float *c, int64_t c_step, int64_t ldc, int M, int part_n, int K, bool two_terms,
-                  int nb, hipStream_t st)
+                  int nb, hipStream_t st, const float *gate = nullptr, int64_t gate_stride = 0,
+                  int S = 0)
 {
     FaArgs g{};
     g.a = a;
@@ -548,14 +579,21 @@ bool launch_parts(const float *a, int64_t lda, const uint16_t *const *w, int par
     g.part_n = part_n;
     g.tiles_n = (g.N + 32 * nb - 1) / (32 * nb);
     g.chunks = K / kFaBK;
+    g.gate = gate;
+    g.gate_stride = gate_stride;
+    g.S = S;
     const int64_t tiles = int64_t((M + kFaBM - 1) / kFaBM) * g.tiles_n;
     if (tiles > INT32_MAX)
         return fail("gemm_f32a: problem too large for one launch");
-    const auto kernel = !two_terms ? gemm_f32a_kernel<1, false, 8>
-                        : nb == 5  ? gemm_f32a_kernel<2, false, 5>
-                        : nb == 6  ? gemm_f32a_kernel<2, false, 6>
-                        : nb == 7  ? gemm_f32a_kernel<2, false, 7>
-                                   : gemm_f32a_kernel<2, false, 8>;
+    const auto pick = [&](auto n5, auto n6, auto n7, auto n8) {
+        return nb == 5 ? n5 : nb == 6 ? n6 : nb == 7 ? n7 : n8;
+    };
+    const auto kernel =
+        !two_terms ? gemm_f32a_kernel<1, false, 8>
+        : gate     ? pick(gemm_f32a_kernel<2, false, 5, true>, gemm_f32a_kernel<2, false, 6, true>,
+                          gemm_f32a_kernel<2, false, 7, true>, gemm_f32a_kernel<2, false, 8, true>)
+                   : pick(gemm_f32a_kernel<2, false, 5>, gemm_f32a_kernel<2, false, 6>,
+                          gemm_f32a_kernel<2, false, 7>, gemm_f32a_kernel<2, false, 8>);
     hipLaunchKernelGGL(kernel, dim3(unsigned(tiles)), dim3(kFaWaves * 64), 0, st, g);
     return hip_ok(hipGetLastError(), "gemm_f32a_kernel launch");
 }
@@ -569,6 +607,20 @@ bool launch_gemm_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t ld
     // One term is bound by its copies, which narrower tiles repeat.
     return launch_parts(a, lda, &w, 1, ldw, c, 0, ldc, M, N, K, two_terms,
                         two_terms ? best_nb(M, N) : kFaNB, st);
+}
+
+// x += gate * (a W^T) without the round trip of the product and the residual
+// pass.  The epilogue's reads of x are exposed, so half of the pass's 19 us at
+// most is gained: sub-layer of 2 x 2304 tokens f32x3 576 -> 571 us, 2 x 4096
+// 1168 -> 1156, 1 x 2704 f32 802 -> 792; 4096 tokens even.
+bool launch_gemm_f32a_residual(const float *a, int64_t lda, const uint16_t *w, int64_t ldw,
+                               float *x, int64_t ldx, const float *gate, int64_t gate_stride,
+                               int S, int M, int N, int K, hipStream_t st)
+{
+    if (!gemm_f32a_fits(M, N, K, lda, ldw, ldx, a, w, x) || !gate || S < 32 || M % S)
+        return fail("gemm_f32a: unsupported shape or alignment (residual)");
+    return launch_parts(a, lda, &w, 1, ldw, x, 0, ldx, M, N, K, true, best_nb(M, N), st, gate,
+                        gate_stride, S);
 }
 
 bool gemm_f32a_three_supported(int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
