@@ -99,12 +99,13 @@ __global__ __launch_bounds__(kGemmWaves * 64, 1) void gemm_bf16_kernel(GemmArgs 
     const int col = lane & 31, half = lane >> 5;
     const int wm = wave & 1, wn = (wave >> 1) & 1, ks = wave >> 2;
 
-    // Tile order: consecutive ids (one XCD) share the split and the A rows.
+    // Tile order: the M tiles (at most 8) of one N tile are consecutive, so an
+    // XCD's 32 workgroups read a near-square block of tiles through its L2.
     const int blk = xcd_major_block();
-    const int tn = blk % g.tiles_n;
-    const int rest = blk / g.tiles_n;
-    const int tm = rest % g.tiles_m;
-    const int sp = rest / g.tiles_m;
+    const int tm = blk % g.tiles_m;
+    const int rest = blk / g.tiles_m;
+    const int tn = rest % g.tiles_n;
+    const int sp = rest / g.tiles_n;
     const int row0 = tm * BM, col0 = tn * BN;
     const int total = g.chunks;
 

@@ -69,6 +69,7 @@ constexpr int kFaStage = kFaAEl + kFaWEl;        // 48 KiB
 constexpr int kFaACopies = kFaAEl / 512 / kFaWaves;  // 1 KiB windows per wave: 4
 constexpr int kFaWCopies = kFaWEl / 512 / kFaWaves;  // most W windows per wave: 2
 constexpr int kFaNB = kFaBN / 32;                // accumulator blocks per wave, widest tile
+constexpr int kFaGroup = 8;                      // tile columns of a group (tile order)
 
 // The attention operands written in place of C by the fused q/k/v
 // projection (launch_gemm_f32a_qkv): columns [0, HD) are q, [HD, 2HD) k,
@@ -91,7 +92,7 @@ struct FaArgs {
     const u16 *w[3];
     float *c;         // [M][ldc]
     int64_t lda, ldw, ldc, c_step;
-    int M, N, part_n, tiles_n, chunks;
+    int M, N, part_n, tiles_m, tiles_n, chunks;
     FaQkv qkv;        // QKV kernels only
     // Residual kernels only: c is the residual x, c[m][n] += gate[m / S][n] * C.
     const float *gate;  // rows gate_stride apart
@@ -293,7 +294,12 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
     const int col = lane & 31, half = lane >> 5;
 
     const int blk = xcd_major_block();
-    const int tn = blk % g.tiles_n, tm = blk / g.tiles_n;
+    // Column groups of 8 tiles, row by row: an XCD's 32 workgroups read a block of
+    // 4 x 8 tiles through its L2.
+    const int group = blk / (g.tiles_m * kFaGroup);
+    const int width = min(kFaGroup, g.tiles_n - group * kFaGroup);
+    const int at = blk - group * g.tiles_m * kFaGroup;
+    const int tm = at / width, tn = group * kFaGroup + at - tm * width;
     const int row0 = tm * kFaBM, col0 = tn * BN;
 
     // Copies.  A window i of wave w is window 4w + i of the A part (8 rows
@@ -578,6 +584,7 @@ bool launch_parts(const float *a, int64_t lda, const uint16_t *const *w, int par
     g.N = parts * part_n;
     g.part_n = part_n;
     g.tiles_n = (g.N + 32 * nb - 1) / (32 * nb);
+    g.tiles_m = (g.M + kFaBM - 1) / kFaBM;
     g.chunks = K / kFaBK;
     g.gate = gate;
     g.gate_stride = gate_stride;
@@ -671,6 +678,7 @@ bool launch_gemm_f32a_qkv(const float *a, int64_t lda, const uint16_t *const w[3
     g.N = 3 * p.H * 128;
     g.part_n = p.H * 128;
     g.tiles_n = g.N / kFaBN;
+    g.tiles_m = (g.M + kFaBM - 1) / kFaBM;
     g.chunks = K / kFaBK;
     g.qkv.qo = p.qo;
     g.qkv.ko = p.ko;
