@@ -100,7 +100,9 @@ __global__ __launch_bounds__(kGemmWaves * 64, 1) void gemm_bf16_kernel(GemmArgs 
     const int wm = wave & 1, wn = (wave >> 1) & 1, ks = wave >> 2;
 
     // Tile order: the M tiles (at most 8) of one N tile are consecutive, so an
-    // XCD's 32 workgroups read a near-square block of tiles through its L2.
+    // XCD's 32 workgroups read a near-square block of tiles through its L2 (two
+    // f32x3 sampler steps at M = 512: 13.61 ms with the N tiles consecutive, 13.47
+    // so).
     const int blk = xcd_major_block();
     const int tm = blk % g.tiles_m;
     const int rest = blk / g.tiles_m;

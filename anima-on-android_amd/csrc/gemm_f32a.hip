@@ -295,7 +295,8 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
 
     const int blk = xcd_major_block();
     // Column groups of 8 tiles, row by row: an XCD's 32 workgroups read a block of
-    // 4 x 8 tiles through its L2.
+    // 4 x 8 tiles through its L2 (24 W blocks and 1.3 A blocks of a row by row
+    // order over 24 columns: 4608 x 6144 x 2048 205.3 us, 200.4 so).
     const int group = blk / (g.tiles_m * kFaGroup);
     const int width = min(kFaGroup, g.tiles_n - group * kFaGroup);
     const int at = blk - group * g.tiles_m * kFaGroup;
