@@ -143,7 +143,9 @@ bool flash_fills_gpu(int64_t BH, int S_q, int D);
 // of a split grid are laid out [splits][BH][S_q][128] f32 and (max, sum) pairs
 // [splits][BH][S_q] float2; those of a balanced grid by slots of 256 rows,
 // slot t + g for tail tile t and share g (along the list either t or g rises
-// by one from part to part).  The max is in log2 units of the scaled scores.
+// by one from part to part).  The max is in log2 units of the scaled scores; the
+// sum is 0 where every score of the part was masked and NaN where one was NaN,
+// whatever the max.
 struct FlashSplitArgs {
     int n = 1;
     int tiles = 1 << 30;

@@ -334,7 +334,7 @@ __global__ __launch_bounds__(NW * 64, 1) void flash_f32_d128(F32Args a, Deal dea
             op = a.split.part + prow * kD;
             tp = nullptr;
             if (half == 0)
-                a.split.ml[prow] = make_float2(m, dead ? 0.0f : l);
+                a.split.ml[prow] = make_float2(m, l);
         }
 #pragma unroll
         for (int r = 0; r < 16; ++r) {

@@ -59,9 +59,10 @@ struct KeysArgs {
     float eps;
 };
 
-// A part with any sum but zero takes part in the merge, a NaN sum included (by
-// bits: this file is compiled without NaN comparisons).
+// By bits: this file is compiled without NaN comparisons.  A part with any sum but
+// zero takes part in the merge, a NaN sum included.
 __device__ __forceinline__ bool joins(const float2 &p) { return (__float_as_uint(p.y) << 1) != 0; }
+__device__ __forceinline__ bool is_nan(float x) { return (__float_as_uint(x) << 1) > 0xFF000000u; }
 
 // The terms of the workgroup's 64 raw rows, bit for bit those of the row prologue
 // (prologue.hip) and q_terms_from_raw: one lane per row adds the squares in
@@ -371,13 +372,14 @@ __global__ __launch_bounds__(512, 1) void flash_keys_d128(KeysArgs a)
         ring_barrier();  // the next K is there, V^T is read
     }
 
-    // Merge the four parts of every row: a part whose max never left -inf saw
-    // masked or NaN scores only and drops out; a NaN sum joins and makes the
-    // row NaN, as in the reference.
+    // Merge the four parts of every row.  A part without a live key has sum 0 and
+    // drops out; a NaN sum joins and makes the row NaN, also where all of the
+    // part's scores were NaN and its max is still -inf; a row whose every part's
+    // max is -inf is zeros, as in the reference (store_o_rows).
     l += l2;
     l += __shfl_xor(l, 32);
     if (half == 0)
-        ml[wave][col] = make_float2(m, m == -INFINITY ? 0.0f : l);
+        ml[wave][col] = make_float2(m, l);
     __syncthreads();
     float mx = -INFINITY;
 #pragma unroll
@@ -388,7 +390,7 @@ __global__ __launch_bounds__(512, 1) void flash_keys_d128(KeysArgs a)
     }
     const float w = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mx);
     if (half == 0)
-        sums[wave][col] = m == -INFINITY ? 0.0f : l * w;
+        sums[wave][col] = mx == -INFINITY ? 0.0f : m == -INFINITY ? l : l * w;
     float *const part = reinterpret_cast<float *>(smem);
 #pragma unroll
     for (int d = 0; d < 4; ++d)
@@ -415,7 +417,7 @@ __global__ __launch_bounds__(512, 1) void flash_keys_d128(KeysArgs a)
             v += *reinterpret_cast<const f32x4 *>(part + ((2 * g + r0) * 32 + rr) * kPitch +
                                                   4 * c4);
         }
-        v *= sum > 0.0f ? 1.0f / sum : 0.0f;  // a NaN sum has NaN in v
+        v *= is_nan(sum) ? sum : sum > 0.0f ? 1.0f / sum : 0.0f;
         const int q = q0 + r;
         store_out4(v, a.o + b * a.ob + h * a.oh + int64_t(q) * a.os,
                    a.ot.t ? a.ot.t + b * a.ot.tb + h * a.ot.th + int64_t(q) * a.ot.ts : nullptr,

@@ -78,9 +78,9 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(CombineArgs a)
 #pragma unroll
         for (int u = 0; u < kU; ++u)
             v[u] = s0 + u < n ? a.sa.ml[(s0 + u) * plane + row0] : make_float2(0.f, 0.f);
-        // A split with l == 0 saw no key (causal) or only masked or NaN
-        // scores; a NaN l (a NaN score among finite ones) joins and makes
-        // the row NaN, as in the reference.
+        // A part with l == 0 saw no key (causal) or only masked ones; a NaN l (a
+        // NaN score, also where the part's live scores are all NaN and its max is
+        // still -inf) joins and makes the row NaN, as in the reference.
 #pragma unroll
         for (int u = 0; u < kU; ++u)
             if (v[u].y != 0.0f)
@@ -109,6 +109,8 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(CombineArgs a)
         }
     }
     const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f;
+    if (mx == -INFINITY)  // no part has a score above -inf: zeros (store_o_rows)
+        acc = f32x4{0.f, 0.f, 0.f, 0.f};
     const int b = int(bh / a.H), h = int(bh - int64_t(b) * a.H);
     flash_tile::store_out4(acc * inv, a.o + b * a.ob + h * a.oh + q * a.os,
                            a.ot.t ? a.ot.t + b * a.ot.tb + h * a.ot.th + q * a.ot.ts : nullptr,

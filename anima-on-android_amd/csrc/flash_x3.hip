@@ -377,7 +377,7 @@ __global__ __launch_bounds__(NW * 64, 1) void flash_x3_d128(X3Args a, Deal deal)
         op = a.split.part + prow0 * kD;
         ostride = kD;
         if (half == 0 && qrow < a.S_q)
-            a.split.ml[prow0 + col] = make_float2(m, dead ? 0.0f : l);
+            a.split.ml[prow0 + col] = make_float2(m, l);
     }
     // Every wave has passed the loop's last barrier: the rings are free.
     store_o_rows(reinterpret_cast<float *>(smem) + wave * kOWaveFloats, o0, o1, o2, o3, inv, dead,
