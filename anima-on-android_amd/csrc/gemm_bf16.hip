@@ -99,15 +99,17 @@ __global__ __launch_bounds__(kGemmWaves * 64, 1) void gemm_bf16_kernel(GemmArgs 
     const int col = lane & 31, half = lane >> 5;
     const int wm = wave & 1, wn = (wave >> 1) & 1, ks = wave >> 2;
 
-    // Tile order: the M tiles (at most 8) of one N tile are consecutive, so an
-    // XCD's 32 workgroups read a near-square block of tiles through its L2 (two
-    // f32x3 sampler steps at M = 512: 13.61 ms with the N tiles consecutive, 13.47
-    // so).
+    // Tile order: consecutive ids (one XCD) share the split and the A rows.  The
+    // other way round (the M tiles of one N tile consecutive, near-square blocks
+    // of tiles per XCD) whole f32x3 calls took, with weights from HBM, 192 x 2048 x
+    // 1024 17.7 against 16.6 us so, 640 x 2048 x 2048 28.2 against 26.5, 512 x 6144
+    // x 2048 35.9 against 34.7, 640 x 8192 x 2048 68.3 against 63.6; at K = 8192
+    // and up to 512 rows the two are even within 1 %.
     const int blk = xcd_major_block();
-    const int tm = blk % g.tiles_m;
-    const int rest = blk / g.tiles_m;
-    const int tn = rest % g.tiles_n;
-    const int sp = rest / g.tiles_n;
+    const int tn = blk % g.tiles_n;
+    const int rest = blk / g.tiles_n;
+    const int tm = rest % g.tiles_m;
+    const int sp = rest / g.tiles_m;
     const int row0 = tm * BM, col0 = tn * BN;
     const int total = g.chunks;
 
