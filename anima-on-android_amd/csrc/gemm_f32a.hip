@@ -512,7 +512,7 @@ __global__ __launch_bounds__(kFaWaves * 64, 1) void gemm_f32a_kernel(FaArgs g)
 
 namespace {
 // Predicted time (us at K = 2048) of the two-term product in 256 x 32 nb tiles on
-// 256 CUs, fitted to 23 shapes of 1100 to 8192 rows on MI355X (within 6 %): a
+// 256 CUs, fitted to shapes of 1100 to 8192 rows on MI355X (within 6 %): a
 // full round is bound by power; one that fills part of the CUs clocks higher
 // until a tile's own copies and latencies bound it.
 double tiles_us(int64_t tiles_m, int64_t N, int nb)
@@ -537,9 +537,12 @@ int best_nb(int M, int N)
 }
 }  // namespace
 
-double gemm_f32a_us(int M, int N)
+// 5 us of it are not in the K loop (1040 to 4032 rows, N = 1024 .. 8192: within
+// 3 % rms from K = 512 to 8192).
+double gemm_f32a_us(int M, int N, int K)
 {
-    return tiles_us((int64_t(M) + kFaBM - 1) / kFaBM, N, best_nb(M, N));
+    const double us = tiles_us((int64_t(M) + kFaBM - 1) / kFaBM, N, best_nb(M, N));
+    return 5.0 + (us - 5.0) * K / 2048;
 }
 
 // Shapes the kernel takes: K a multiple of 32, 16-byte aligned A and W rows,

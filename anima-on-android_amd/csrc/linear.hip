@@ -309,12 +309,17 @@ size_t linear_scratch_bytes(int M, int K, bool exact)
 }
 
 // Always where 256 x 256 tiles fill the GPU.  Below that, past the small-M
-// kernel's rows, where its prediction beats those of the other ways by 4 % (at
-// K = 2048, us, fitted to the same shapes): the 128 x 256 kernel where its
-// tiles fill the GPU (62 a round, a last round of at least 40: 4096 x 2048 62
-// against 72 here, 4608 x 2048 102 against 75), or the split pass and two
-// library products (16 plus 0.9 PFLOP/s: 2048 x 2048 54 against 60, 3584 x
-// 2048 76 against 67, 1536 x 6144 103 against 76).
+// kernel's rows, where its prediction beats those of the other ways by 4 %:
+//   * the 128 x 256 kernel where its tiles fill the GPU (us at K = 2048: 62 a
+//     round, a last round of at least 40; 4 of that is not in the K loop: 4096 x
+//     2048 62 against 72 here, 4608 x 2048 102 against 75);
+//   * the split pass and two library products: 20 us, 0.002 a k, and 1.15
+//     PFLOP/s.  That comes to within 9 % on 155 shapes of 1040 to 4032 rows, N =
+//     1024 .. 8192 and K = 512 .. 8192, and this kernel took none of them where
+//     it was more than 1 % behind.  Measured, the library's way against this
+//     kernel's: 2560 x 2048 at K = 512 32 against 20, at 2048 58 against 60, at
+//     8192 177 against 226; 3840 x 2048 40 against 22, 77 against 67, 253
+//     against 249; 1040 x 6144 36 against 21, 66 against 65, 208 against 248.
 bool linear_takes_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, const float *c,
                        int64_t ldc, int M, int N, int K)
 {
@@ -322,13 +327,15 @@ bool linear_takes_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t l
         return true;
     if (!gemm_f32a_fits(M, N, K, lda, ldw, ldc, a, w, c) || small_m_path(M, K, true))
         return false;
-    double other = 16.0 + 4.0 * M * double(N) * 2048 / 0.9e9;
+    double other = 20.0 + (4.0 * M * double(N) / 1.15e9 + 0.002) * K;
     if (gemm_large_f32a_supported(M, N, K, lda, ldw, ldc, a, w, c)) {
         const int64_t tiles = ((int64_t(M) + 127) / 128) * ((int64_t(N) + 255) / 256);
         const int64_t rest = tiles % 256;
-        other = double(tiles / 256) * 62.0 + (rest ? std::max(40.0, 0.24 * double(rest)) : 0.0);
+        const double us =
+            double(tiles / 256) * 62.0 + (rest ? std::max(40.0, 0.24 * double(rest)) : 0.0);
+        other = 4.0 + (us - 4.0) * K / 2048;
     }
-    return 1.04 * gemm_f32a_us(M, N) <= other;
+    return 1.04 * gemm_f32a_us(M, N, K) <= other;
 }
 
 bool launch_linear(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, float *c,

@@ -301,8 +301,8 @@ bool anima_hip_gemm_dev(const float *a, int64_t lda, const void *w, int w_bf16, 
  * split-K partials of the hand-written small-M GEMM, which then runs instead
  * of the library GEMM; the partials are added in a fixed order, so results
  * are deterministic.  At larger M (K a multiple of 32, 16-byte aligned A rows
- * with lda % 4 == 0) the f32 modes where M x N is about 2700 x 2048 or more,
- * and the bf16 mode where a grid has at least 256 tiles of 256 x 256 and N and
+ * with lda % 4 == 0) the f32 modes where M x N is large for K (about 2700 x 2048
+ * or more at K = 2048, 3800 x 2048 at K = 8192), and the bf16 mode where a grid has at least 256 tiles of 256 x 256 and N and
  * K are at most 2048, run a kernel that stages the f32 rows of a and splits (or
  * rounds) them in registers (in the f32 modes bit-identical to the split pass
  * followed by the hand-written product on the term rows).  Shapes without a

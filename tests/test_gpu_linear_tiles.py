@@ -42,7 +42,7 @@ def run(a, w, M, N, K, lda):
 # (1100 x 8192); one to six chunks of K; ragged last rows.  The kernel on term
 # rows takes K in multiples of 64.
 @pytest.mark.parametrize("M,N,K,same_bits", [
-    (1536, 6144, 32, False), (1100, 8192, 64, True), (4352, 2048, 192, True),
+    (1536, 6144, 32, False), (1100, 8192, 192, True), (4352, 2048, 192, True),
     (2700, 2040, 128, False), (2700, 8192, 64, True), (3333, 6140, 96, False),
     (4552, 8192, 64, True), (3016, 8100, 128, True)])
 def test_tile_widths(M, N, K, same_bits):
