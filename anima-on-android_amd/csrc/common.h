@@ -3,7 +3,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
-#include "flash_deal.h"
+#include "flash_plan.h"
 #include <cstdint>
 #include <string>
 
@@ -65,79 +65,6 @@ struct FlashProblem {
     RawQ rq;           // f32x3, f32 and bf16 kernels: q given as raw projection rows
 };
 bool term_out_ok(const TermOut &t);  // alignment of a set term output
-
-// Launch shape of the D == 128 flash kernels: T = B*H*ceil(S_q/256) query
-// tiles of 8-wave workgroups, or twice as many of 4 waves, over n key tiles of
-// 64 keys, on 256 CUs that hold one workgroup each.  Five shapes:
-//   whole     8-wave workgroups, one query tile each;
-//   small     4-wave workgroups, one query tile each (T < 256);
-//   split     4-wave workgroups, the key range of every query tile split over
-//             `splits` of them ("split-KV"): split s takes key tiles
-//             [s*tiles, (s+1)*tiles);
-//   balanced  the largest multiple of 256 query tiles whole, and the key tiles
-//             of the `ntail` others as one list dealt out evenly, `u` to each
-//             of the last workgroups (T = 288 over 36 key tiles: 36 + 5 tiles
-//   keys      (bf16 MFMA) 8-wave workgroups of 64 query rows whose waves share
-//             the keys among them (flash_keys.hip): at most 256 of them.
-// A workgroup that sees part of a query tile's keys writes its output
-// normalised by its own row sum, plus that row's (max, sum), to scratch, and
-// flash_combine merges the parts into O.
-struct FlashPlan {
-    bool keys = false;    // the keys shape
-    int waves = 8;
-    int splits = 1;
-    int tiles = 1 << 30;  // key tiles per split
-    int full = 0;         // balanced: query tiles run whole
-    int ntail = 0;        // balanced: query tiles dealt out
-    int nk = 0;           // balanced: key tiles of a query tile
-    int u = 0;            // balanced: key tiles per workgroup (0: another shape)
-    size_t bytes = 0;     // scratch for the partials (0 when every tile runs whole)
-};
-// What a kernel takes per 64-key tile (us) in a 4-wave and in an 8-wave
-// workgroup when every CU holds one, measured on MI355X (4-wave: 32 heads x
-// 256 queries, unsplit grids over 4 and 8 key tiles; 8-wave: 32 heads x 4096
-// queries and keys).  The bf16-MFMA kernels are bound by power: an 8-wave
-// round of at most about 0.7 of the CUs clocks higher, down to `part` of w8
-// (x3, T = 288 .. 800: 0.66 .. 0.76 of the full rounds' time per tile); the
-// f32 MFMA runs at full clock either way.
-// The keys shape: `round` for every 64 KiB of K that its four key groups take
-// together (keys_round of them), and `merge` once, both against what a 4-wave
-// workgroup spends beside its tiles (256 and 1024 queries and keys, 16 heads;
-// 0: the mode has no such kernel).
-struct FlashTimes {
-    float w4, w8, part, merge, round;
-    int keys_round;
-};
-constexpr FlashTimes kTimesF32{9.1f, 15.7f, 1.0f, 0.0f, 0.0f, 0},
-    kTimesBF16{1.3f, 1.9f, 0.7f, 1.5f, 2.8f, 256}, kTimesX3{2.5f, 4.6f, 0.7f, 1.0f, 3.2f, 128};
-// Fixed cost (us) of split grids and of balanced ones, whose parts are twice
-// as tall: every part loads its query tile and writes f32 partials, which the
-// combine pass reads back (25 to 31 us at T = 144 and 288, every mode).
-constexpr float kSplitCostUs = 13.0f, kBalanceCostUs = 27.0f;
-// Scratch a flash launch may use, 16-byte aligned; either may be null.
-struct FlashScratch {
-    void *part = nullptr;
-    size_t part_bytes = 0;
-    void *balance = nullptr;
-    size_t balance_bytes = 0;
-    bool keys = false;  // the keys shape may run (the caller needs no other shape's bits)
-    // What it saves (us) because it alone takes the query rows raw: a row pass
-    // of its own before the kernel.
-    float keys_saves = 0.0f;
-};
-
-// The shape with the least predicted time among those whose partials fit:
-// s.part_bytes for `split`, s.balance_bytes for `balanced` (causal calls, whose
-// tiles differ in length, are not balanced, and `keys` has no mask).
-FlashPlan flash_plan(int64_t BH, int S_q, int S_kv, int D, const FlashTimes &t, bool causal,
-                     const FlashScratch &s);
-// Scratch that holds the partials of a split grid in every mode, and that of
-// a balanced grid (0 where none would run).
-size_t flash_split_bytes(int64_t BH, int S_q, int S_kv, int D);
-size_t flash_balance_bytes(int64_t BH, int S_q, int S_kv, int D, const FlashTimes &t);
-constexpr size_t kMaxFlashBalanceBytes = size_t(511) * 256 * (128 * 4 + 8);  // 65 MiB
-// A grid of 8-wave workgroups with at least one for each CU.
-bool flash_fills_gpu(int64_t BH, int S_q, int D);
 
 // What a workgroup that sees part of the keys writes (device view).  Partials
 // of a split grid are laid out [splits][BH][S_q][128] f32 and (max, sum) pairs

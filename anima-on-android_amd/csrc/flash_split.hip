@@ -1,6 +1,5 @@
-// Launch plans of the D == 128 flash kernels (which query tiles run whole and
-// whose keys are shared out over several workgroups) and the kernel that
-// merges the partial outputs.
+// The kernel that merges the partial outputs of the D == 128 flash kernels where
+// a query tile's keys are shared out over several workgroups (flash_plan.h).
 //
 // Merging follows from the online-softmax identity the flash kernels already
 // use between key tiles (anima_rt/include/cpu/flash_attention.h:145-178 rescales
@@ -18,14 +17,7 @@ namespace {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int kD = 128;
-constexpr int kBN = 64;            // keys per tile of the flash kernels
-constexpr int kTargetBlocks = kFlashTargetBlocks;
-constexpr int kBM8 = 256;          // query rows of an 8-wave workgroup
-constexpr size_t kSlotBytes = size_t(kBM8) * (kD * sizeof(float) + sizeof(float2));
-
-int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
-size_t round_up256(size_t n) { return (n + 255) / 256 * 256; }
+constexpr int kD = kFlashD, kBM8 = kFlashRows8;
 
 struct CombineArgs {
     float *o;
@@ -125,116 +117,6 @@ bool term_out_ok(const TermOut &t)
            t.ts % 8 == 0 && t.lo % 8 == 0 && t.lo >= 0;
 }
 
-namespace {
-
-// The split shape, which every mode's scratch must hold: 4-wave workgroups,
-// the key range over ~256 of them.
-FlashPlan split_plan(int64_t BH, int S_q, int S_kv, int D)
-{
-    FlashPlan pl;
-    if (D != kD || BH <= 0 || S_q <= 0 || BH * ceil_div(S_q, kBM8) >= kTargetBlocks)
-        return pl;
-    pl.waves = 4;
-    const int64_t units = BH * ceil_div(S_q, 128);
-    const int64_t ntiles = ceil_div(S_kv, kBN);
-    const int64_t want = ceil_div(kTargetBlocks, units);
-    if (want < 2 || ntiles < 2)
-        return pl;
-    const int64_t tiles = ceil_div(ntiles, std::min(want, ntiles));
-    const int64_t splits = ceil_div(ntiles, tiles);
-    if (splits < 2)
-        return pl;
-    pl.splits = int(splits);
-    pl.tiles = int(tiles);
-    const size_t rows = size_t(splits) * size_t(BH) * size_t(S_q);
-    pl.bytes = round_up256(rows * kD * sizeof(float)) + rows * sizeof(float2);
-    return pl;
-}
-
-// The balanced shape; u == 0 where the query tiles come out even, or where a
-// share would be a whole tile anyway.
-FlashPlan balanced_plan(int64_t BH, int S_q, int S_kv, int D)
-{
-    FlashPlan pl;
-    if (D != kD || BH <= 0 || S_q <= 0 || S_kv <= 0)
-        return pl;
-    const int64_t T = BH * ceil_div(S_q, kBM8), nk = ceil_div(S_kv, kBN);
-    const int64_t tail = T % kTargetBlocks;
-    if (tail == 0 || T > INT32_MAX / 2 || nk > INT32_MAX / kTargetBlocks)
-        return pl;
-    const int64_t u = ceil_div(tail * nk, kTargetBlocks);
-    if (u >= nk)
-        return pl;
-    pl.full = int(T - tail);
-    pl.ntail = int(tail);
-    pl.nk = int(nk);
-    pl.u = int(u);
-    pl.bytes = size_t(tail + ceil_div(tail * nk, u) - 1) * kSlotBytes;
-    return pl;
-}
-
-}  // namespace
-
-FlashPlan flash_plan(int64_t BH, int S_q, int S_kv, int D, const FlashTimes &t, bool causal,
-                     const FlashScratch &s)
-{
-    FlashPlan best;
-    if (D != kD || BH <= 0 || S_q <= 0)
-        return best;
-    const int64_t T = BH * ceil_div(S_q, kBM8), T4 = BH * ceil_div(S_q, 128);
-    const double n = double(ceil_div(S_kv, kBN));
-    const auto rounds = [](int64_t blocks) { return double(ceil_div(blocks, kTargetBlocks)); };
-    // Whole rounds of 8-wave workgroups, and one that fills part of the CUs.
-    const double tail = double(T % kTargetBlocks) / kTargetBlocks;
-    double us = (double(T / kTargetBlocks) + (tail > 0 ? std::max(tail, double(t.part)) : 0)) * n *
-                t.w8;
-    const auto consider = [&](const FlashPlan &pl, double cost) {
-        if (cost < us) {
-            us = cost;
-            best = pl;
-        }
-    };
-    if (T < kTargetBlocks) {
-        FlashPlan small;
-        small.waves = 4;
-        consider(small, rounds(T4) * n * t.w4);
-        const FlashPlan sp = split_plan(BH, S_q, S_kv, D);
-        if (sp.splits > 1 && sp.bytes <= s.part_bytes)
-            consider(sp, rounds(T4 * sp.splits) * sp.tiles * t.w4 + kSplitCostUs);
-    }
-    const FlashPlan bal = balanced_plan(BH, S_q, S_kv, D);
-    if (bal.u > 0 && !causal && bal.bytes <= s.balance_bytes)
-        consider(bal, (bal.full / kTargetBlocks * n + bal.u) * t.w8 + kBalanceCostUs);
-    // One key tile of 64 has nothing to share (64 queries and keys, 16 heads:
-    // 14.1 us whole against 16.1), and a second round of workgroups loses to
-    // the taller tiles (576 queries and keys, 32 heads, f32x3: 46 against 60).
-    if (s.keys && t.keys_round > 0 && !causal && S_kv > kBN &&
-        BH * ceil_div(S_q, 64) <= kTargetBlocks) {
-        FlashPlan keys;
-        keys.keys = true;
-        consider(keys, t.merge + ceil_div(S_kv, t.keys_round) * t.round - s.keys_saves);
-    }
-    return best;
-}
-
-size_t flash_split_bytes(int64_t BH, int S_q, int S_kv, int D)
-{
-    return split_plan(BH, S_q, S_kv, D).bytes;
-}
-
-size_t flash_balance_bytes(int64_t BH, int S_q, int S_kv, int D, const FlashTimes &t)
-{
-    FlashScratch any;
-    any.part_bytes = any.balance_bytes = SIZE_MAX;
-    const FlashPlan pl = flash_plan(BH, S_q, S_kv, D, t, false, any);
-    return pl.u > 0 ? pl.bytes : 0;
-}
-
-bool flash_fills_gpu(int64_t BH, int S_q, int D)
-{
-    return D != kD || BH <= 0 || S_q <= 0 || BH * ceil_div(S_q, kBM8) >= kTargetBlocks;
-}
-
 FlashSplitArgs flash_split_args(const FlashPlan &pl, int64_t BH, int S_q, const FlashScratch &s,
                                 FlashDeal &deal)
 {
@@ -248,7 +130,7 @@ FlashSplitArgs flash_split_args(const FlashPlan &pl, int64_t BH, int S_q, const 
         sa.u = pl.u;
         deal_pieces(pl.ntail, pl.nk, pl.u, deal, sa.ng, sa.nshorter);
         sa.part = static_cast<float *>(s.balance);
-        rows = pl.bytes / kSlotBytes * kBM8;
+        rows = pl.bytes / kFlashSlotBytes * kBM8;
     } else if (pl.splits > 1) {
         sa.n = pl.splits;
         sa.tiles = pl.tiles;
@@ -256,7 +138,7 @@ FlashSplitArgs flash_split_args(const FlashPlan &pl, int64_t BH, int S_q, const 
         rows = size_t(pl.splits) * size_t(BH) * size_t(S_q);
     }
     sa.ml = reinterpret_cast<float2 *>(reinterpret_cast<char *>(sa.part) +
-                                       round_up256(rows * kD * sizeof(float)));
+                                       flash_round_up256(rows * kD * sizeof(float)));
     return sa;
 }
 
@@ -264,7 +146,7 @@ int64_t flash_blocks(const FlashSplitArgs &sa, int64_t BH, int S_q, int BM)
 {
     if (sa.u > 0)
         return sa.full + sa.ng + sa.nshorter;
-    return BH * ceil_div(S_q, BM) * sa.n;
+    return BH * flash_ceil_div(S_q, BM) * sa.n;
 }
 
 bool launch_flash_combine(const FlashProblem &p, const FlashSplitArgs &sa, hipStream_t st)
@@ -276,12 +158,12 @@ bool launch_flash_combine(const FlashProblem &p, const FlashSplitArgs &sa, hipSt
     a.os = p.os.s;
     a.H = p.H;
     a.S_q = p.S_q;
-    a.n_qtiles = int(ceil_div(p.S_q, kBM8));
+    a.n_qtiles = int(flash_ceil_div(p.S_q, kBM8));
     a.sa = sa;
     a.ot = p.ot;
     const bool bal = sa.u > 0;
     a.total = (bal ? int64_t(sa.ntail) * kBM8 : sa.BH * p.S_q) * (kD / 4);
-    const int64_t nblk = ceil_div(a.total, 256);
+    const int64_t nblk = flash_ceil_div(a.total, 256);
     if (nblk > INT32_MAX)
         return fail("flash_combine: problem too large for one launch");
     if (bal)

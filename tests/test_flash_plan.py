@@ -1,0 +1,53 @@
+"""The launch shape of a flash attention (csrc/flash_plan.h), asked for on the CPU
+through tests/native/flash_plan_shape.cpp: the shapes that were measured fastest
+where the cost models of two of them come close."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from anima_hip import rt
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+MODES = {rt.F32: "f32", rt.BF16: "bf16", rt.F32X3: "f32x3"}
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+
+
+@pytest.fixture(scope="module")
+def shape(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("plan") / "flash_plan_shape")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fsanitize=undefined", "-fno-sanitize-recover=all",
+                    "-Wall", "-Werror", "-I", os.path.join(ROOT, "anima-on-android_amd", "csrc"),
+                    os.path.join(ROOT, "tests", "native", "flash_plan_shape.cpp"), "-o", exe],
+                   check=True)
+
+    def ask(mode, BH, S_q, S_kv, causal=False, keys=None, saves=0.0):
+        keys = mode != rt.F32 if keys is None else keys
+        line = f"{MODES[mode]} {BH} {S_q} {S_kv} {int(causal)} {int(keys)} {saves}\n"
+        run = subprocess.run([exe], input=line, capture_output=True, text=True, timeout=60)
+        assert run.returncode == 0, run.stdout + run.stderr
+        return run.stdout.strip()
+    return ask
+
+
+# Whole calls of anima_hip_attention_dev in every shape (us): the fastest one, with
+# the next beside it.
+@pytest.mark.parametrize("mode,BH,S_q,S_kv,fastest", [
+    (rt.F32X3, 5, 64, 512, "split"),      # 24.1, keys 29.5
+    (rt.F32X3, 16, 64, 512, "split"),     # 27.6, keys 31.2
+    (rt.F32X3, 5, 256, 385, "split"),     # 26.8, keys 28.5
+    (rt.F32X3, 32, 64, 512, "split"),     # 32.7, keys 36.7
+    (rt.F32X3, 16, 256, 512, "keys"),     # split 1.2 more
+    (rt.F32X3, 16, 256, 256, "keys"),
+    (rt.F32X3, 16, 1024, 1024, "keys"),
+    (rt.F32, 32, 257, 257, "split"),      # 52.2, small 60.5
+    (rt.F32, 32, 320, 320, "split"),      # 52.6, balanced 60.9
+    (rt.F32, 16, 768, 320, "balanced"),
+    (rt.F32, 16, 600, 600, "balanced"),
+    (rt.F32, 5, 64, 65, "split"),         # 21.9, small 27.5
+    (rt.BF16, 5, 256, 1000, "keys"),
+    (rt.BF16, 16, 768, 192, "small")])
+def test_measured_shapes(shape, mode, BH, S_q, S_kv, fastest):
+    assert shape(mode, BH, S_q, S_kv) == fastest
