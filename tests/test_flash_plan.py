@@ -1,16 +1,21 @@
 """The launch shape of a flash attention (csrc/flash_plan.h), asked for on the CPU
 through tests/native/flash_plan_shape.cpp: the shapes that were measured fastest
-where the cost models of two of them come close."""
+where the cost models of two of them come close, and the shape that each case of
+the GPU tests of one shape is there for."""
 import os
 import shutil
 import subprocess
 
 import pytest
 
+import test_gpu_balanced
+import test_gpu_keys
+import test_gpu_nan_parts
 from anima_hip import rt
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 MODES = {rt.F32: "f32", rt.BF16: "bf16", rt.F32X3: "f32x3"}
+RAW_SAVES = 6.0  # attention.hip's kRowPassUs: cached keys, raw query rows
 
 pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
 
@@ -51,3 +56,32 @@ def shape(tmp_path_factory):
     (rt.BF16, 16, 768, 192, "small")])
 def test_measured_shapes(shape, mode, BH, S_q, S_kv, fastest):
     assert shape(mode, BH, S_q, S_kv) == fastest
+
+
+@pytest.mark.parametrize("mode,B,H,S_q,S_kv", test_gpu_keys.CASES)
+def test_keys_cases(shape, mode, B, H, S_q, S_kv):
+    assert shape(mode, B * H, S_q, S_kv) == "keys"
+
+
+@pytest.mark.parametrize("mode", test_gpu_keys.MODES)
+@pytest.mark.parametrize("case", test_gpu_keys.RAW_CASES)
+def test_raw_keys_cases(shape, mode, case):
+    B, S_q, S_kv = case
+    assert shape(mode, 16 * B, S_q, S_kv, saves=RAW_SAVES) == "keys"
+
+
+def test_nan_cases(shape):
+    for mode, S, _ in test_gpu_nan_parts.KEYS:
+        assert shape(mode, 16, S, S) == "keys"
+    for mode in (rt.F32X3, rt.BF16):
+        assert shape(mode, 16, 100, 65, saves=RAW_SAVES) == "keys"
+    for mode, BH, S_q, S_kv, _ in test_gpu_nan_parts.BALANCED:
+        assert shape(mode, BH, S_q, S_kv, keys=False) == "balanced"
+    for mode in MODES:
+        assert shape(mode, 2, 961, 961, keys=False) == "split"
+
+
+def test_balanced_cases(shape):
+    for B, H, S_q, S_kv, modes in test_gpu_balanced.CASES:
+        for mode in modes:
+            assert shape(mode, B * H, S_q, S_kv) == "balanced"

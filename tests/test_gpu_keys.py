@@ -2,7 +2,8 @@
 anima_hip_attention_dev (prepared query rows) and the cached cross-attention
 (raw query rows), against the oracle at the stated tolerances: one ragged query
 tile and a full grid of 256; one key past a tile, key ranges that leave key
-groups idle in the last round, several rounds.
+groups idle in the last round, several rounds.  test_flash_plan.py holds CASES and
+RAW_CASES to the shape they are here for; OTHER runs small grids beside it.
 """
 import ctypes as ct
 
@@ -29,10 +30,16 @@ def _check(out, ref, mode):
     assert err <= (2e-2 * float(np.abs(ref).max()) if mode == rt.BF16 else 1e-4)
 
 
-@pytest.mark.parametrize("mode", MODES)
-@pytest.mark.parametrize("B,H,S_q,S_kv", [(1, 3, 65, 65), (1, 16, 200, 129), (2, 5, 64, 300),
-                                          (1, 16, 1024, 96), (1, 2, 1, 1000)])
-def test_keys_shape(B, H, S_q, S_kv, mode):
+CASES = [(rt.F32X3, 1, 3, 65, 65), (rt.F32X3, 1, 16, 200, 129), (rt.F32X3, 2, 5, 64, 300),
+         (rt.F32X3, 1, 16, 1024, 96), (rt.F32X3, 1, 16, 1000, 1000), (rt.BF16, 1, 2, 1, 1000),
+         (rt.BF16, 1, 16, 200, 193), (rt.BF16, 1, 16, 1024, 250), (rt.BF16, 1, 16, 200, 600),
+         (rt.BF16, 2, 5, 64, 900)]
+OTHER = [(rt.F32X3, 1, 2, 1, 1000), (rt.BF16, 1, 3, 65, 65), (rt.BF16, 1, 16, 200, 129),
+         (rt.BF16, 2, 5, 64, 300), (rt.BF16, 1, 16, 1024, 96)]
+
+
+@pytest.mark.parametrize("mode,B,H,S_q,S_kv", CASES + OTHER)
+def test_keys_shape(mode, B, H, S_q, S_kv):
     from devmem import DevBuf
     lib = _lib.load()
     rng = np.random.default_rng(B + H + S_q + S_kv + mode)
@@ -60,8 +67,11 @@ def test_keys_shape(B, H, S_q, S_kv, mode):
     _check(np.where(nan, 0, got), np.where(nan, 0, ref), mode)
 
 
+RAW_CASES = [(1, 100, 77), (2, 256, 512), (1, 1000, 65)]
+
+
 @pytest.mark.parametrize("mode", MODES)
-@pytest.mark.parametrize("B,S_q,S_kv", [(1, 100, 77), (2, 256, 512), (1, 1000, 65)])
+@pytest.mark.parametrize("B,S_q,S_kv", RAW_CASES)
 def test_keys_shape_raw_queries(B, S_q, S_kv, mode):
     rng = np.random.default_rng(B + S_q + S_kv + 7 * mode)
     H, C = 16, 256
