@@ -33,6 +33,7 @@
 // q/k/v product is the f32-activation kernel's fused form (gemm_f32a.hip),
 // which writes the attention's prepared Q, K and V^T itself.
 #include "common.h"
+#include "gelu_poly.h"
 
 #include "anima_hip.h"
 
@@ -197,29 +198,19 @@ struct GeluArgs {
     unsigned blocks;  // workgroups per row
 };
 
-// x Phi(x) = max(x, 0) - |x| Phi(-|x|), Phi(-t) = exp(-t^2 / 2) P(u) with
-// u = t / (1 + t / 2) and P(0) = 1/2: a polynomial fitted here to
-// erfcx(t / sqrt(2)) / 2 on 0 <= t <= 14 (weighted minimax, exp(-t^2 / 2) times its
-// error <= 1.6e-9).  Against float64 its largest error over normal values of
-// scales 0.05 to 3 and all of [-14, 14] is 2.4e-7 (0.5 x (1 + erff): 4.5e-7),
-// relative to |x| 8.4e-8 (1.05e-7), and the negative tail keeps six digits.
+// x Phi(x) = max(x, 0) - |x| Phi(-|x|), Phi(-t) = exp(-t^2 / 2) P(u) (gelu_poly.h)
+// with u = t / (1 + t / 2).  Against float64 its largest error over normal values
+// of scales 0.05 to 3 and all of [-14, 14] is 2.4e-7 (0.5 x (1 + erff): 4.5e-7),
+// relative to |x| 8.4e-8 (1.05e-7); relative to the value the negative tail is
+// good to 5e-6 down to x = -6 and 4.5e-5 down to -13.
 // t stops at 40 above so that inf gives inf; NaN stays NaN, -inf gives NaN as
 // 0.5 x (1 + erff) does.
 __device__ __forceinline__ float gelu(float x)
 {
     const float t = fabsf(fminf(x, 40.0f));
     const float u = t * __builtin_amdgcn_rcpf(fmaf(t, 0.5f, 1.0f));
-    float p = 1.143050249e-04f;
-    p = fmaf(p, u, -2.704118961e-04f);
-    p = fmaf(p, u, -2.087033645e-04f);
-    p = fmaf(p, u, -1.072004903e-03f);
-    p = fmaf(p, u, 6.642731605e-04f);
-    p = fmaf(p, u, 1.728924364e-02f);
-    p = fmaf(p, u, 5.052748695e-02f);
-    p = fmaf(p, u, -3.989422023e-01f);
-    p = fmaf(p, u, 0.5f);
     const float e = __builtin_amdgcn_exp2f(x * (x * -0.72134752044f));  // exp(-x^2 / 2)
-    return fmaf(-t, p * e, fmaxf(x, 0.0f));
+    return fmaf(-t, gelu_poly(u) * e, fmaxf(x, 0.0f));
 }
 
 template <bool H_BF16>
