@@ -1,8 +1,8 @@
 """The DiT's small kernels at sizes around their workgroups.
 
-The MLP at hidden widths around the GELU pass's workgroups of 2048 values
-(a small row, a row of one group and 8 values, three whole groups) against the
-oracle's model; tolerances of the whole DiT's tests (1e-4 in the f32 mode, 3e-2
+The MLP at hidden widths around the GELU pass's workgroups of 1 to 4 waves of 512
+values (one wave and the next ragged, one workgroup of two, five of one, two of
+three, three of four) against the oracle's model; tolerances of the whole DiT's tests (1e-4 in the f32 mode, 3e-2
 in bf16); and a model of enough blocks that the launches of all AdaLN layers give
 each lane group two rows, at a width whose rows and columns come out ragged."""
 import os
@@ -42,7 +42,7 @@ def check(cfg, mode):
 
 
 @pytest.mark.parametrize("mode", [rt.F32, rt.BF16])
-@pytest.mark.parametrize("hidden", [264, 2056, 6144])
+@pytest.mark.parametrize("hidden", [264, 776, 2056, 3072, 6144])
 def test_mlp_widths(hidden, mode):
     check(dict(dim=256, blocks=2, heads=2, head_dim=128, mlp_hidden=hidden, ctx_dim=64), mode)
 
