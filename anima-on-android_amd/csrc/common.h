@@ -76,20 +76,33 @@ bool term_out_ok(const TermOut &t);  // alignment of a set term output
 struct FlashSplitArgs {
     int n = 1;
     int tiles = 1 << 30;
-    int full = 0, ntail = 0, nk = 1, u = 0;
-    int ng = 0;        // balanced: shares
-    int nshorter = 0;  // balanced: workgroups that take a shorter piece
     int64_t BH = 0;
     float *part = nullptr;
     float2 *ml = nullptr;
 };
-struct FlashWhole {};  // in FlashDeal's place where no query tile is dealt out
+// A balanced grid's tail tiles (FlashPlan), its shares and the workgroups that take
+// a shorter piece; and with them the order of the pieces.  Kernel arguments of the
+// balanced grids alone: a workgroup waits for every line of its arguments, and
+// with these six in FlashSplitArgs the calls on split grids took 0.5 to 0.8 us more.
+struct FlashTail {
+    int full = 0, ntail = 0, nk = 1, u = 0;
+    int ng = 0, nshorter = 0;
+};
+struct FlashShares {
+    FlashTail tail;
+    FlashDeal deal;
+};
+struct FlashWhole {};  // in FlashShares' place where no query tile is dealt out
+// Fills `sh` for a balanced plan (sh.tail.u > 0).
 FlashSplitArgs flash_split_args(const FlashPlan &pl, int64_t BH, int S_q, const FlashScratch &s,
-                                FlashDeal &deal);
+                                FlashShares &sh);
 // Workgroups of the launch: BM query rows per tile.
-int64_t flash_blocks(const FlashSplitArgs &sa, int64_t BH, int S_q, int BM);
-// O[b,h,q,:] = sum_s w_s P_s[bh,q,:] / sum_s w_s, w_s = l_s * 2^(m_s - max_s m_s).
-bool launch_flash_combine(const FlashProblem &p, const FlashSplitArgs &sa, hipStream_t st);
+int64_t flash_blocks(const FlashSplitArgs &sa, const FlashWhole &, int64_t BH, int S_q, int BM);
+int64_t flash_blocks(const FlashSplitArgs &sa, const FlashShares &sh, int64_t BH, int S_q, int BM);
+// O[b,h,q,:] = sum_s w_s P_s[bh,q,:] / sum_s w_s, w_s = l_s * 2^(m_s - max_s m_s),
+// where a launch wrote parts.
+bool launch_flash_combine(const FlashProblem &p, const FlashSplitArgs &sa, const FlashTail &tail,
+                          hipStream_t st);
 
 // f32 inputs, f32 MFMA (D == 128) or the generic kernel (any D <= 1024).
 bool launch_flash_f32(const FlashProblem &p, hipStream_t st, const FlashScratch &scr = {});

@@ -468,7 +468,7 @@ bool launch_d128(const Bf16Args &a, const Deal &deal, int64_t BH, hipStream_t st
     constexpr int BM = NW * 32;
     Bf16Args g = a;
     g.n_qtiles = (g.S_q + BM - 1) / BM;
-    const int64_t nblk = flash_blocks(g.split, BH, g.S_q, BM);
+    const int64_t nblk = flash_blocks(g.split, deal, BH, g.S_q, BM);
     if (nblk > INT32_MAX)
         return fail("flash_bf16: problem too large for one launch");
     hipLaunchKernelGGL((flash_bf16_d128<NW, ST, Deal>), dim3(unsigned(nblk)), dim3(NW * 64), 0, st,
@@ -541,16 +541,16 @@ bool launch_flash_bf16(const FlashProblem &p, hipStream_t st, const FlashScratch
         return launch_flash_keys(p, 1, a.dma32 != 0, st);
     if (p.rq.parts > 1)
         return fail("flash_bf16: this launch shape takes no query planes");
-    FlashDeal deal;
-    a.split = flash_split_args(pl, BH, p.S_q, scr, deal);
+    FlashShares shares;
+    a.split = flash_split_args(pl, BH, p.S_q, scr, shares);
     const FlashWhole whole;
     const bool ok = paired_plan(pl, p.S_kv) ? launch_d128<4, 2>(a, whole, BH, st)
                     : pl.waves == 4        ? launch_d128<4, 3>(a, whole, BH, st)
-                    : pl.u > 0             ? launch_d128<8, 3>(a, deal, BH, st)
+                    : pl.u > 0             ? launch_d128<8, 3>(a, shares, BH, st)
                                            : launch_d128<8, 3>(a, whole, BH, st);
     if (!ok)
         return false;
-    return (a.split.n == 1 && a.split.u == 0) || launch_flash_combine(p, a.split, st);
+    return launch_flash_combine(p, a.split, shares.tail, st);
 }
 
 bool launch_vt_pack(const float *v, Strides vs, uint16_t *vt, Strides vts, int B, int H,

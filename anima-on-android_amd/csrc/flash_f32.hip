@@ -444,7 +444,7 @@ bool launch_d128(const F32Args &a, const Deal &deal, int64_t BH, hipStream_t st)
     constexpr int BM = NW * 32;
     F32Args g = a;
     g.n_qtiles = (g.S_q + BM - 1) / BM;
-    const int64_t nblk = flash_blocks(g.split, BH, g.S_q, BM);
+    const int64_t nblk = flash_blocks(g.split, deal, BH, g.S_q, BM);
     if (nblk > INT32_MAX)
         return fail("flash_f32: problem too large for one launch");
     hipLaunchKernelGGL((flash_f32_d128<NW, Deal>), dim3(unsigned(nblk)), dim3(NW * 64), 0, st, g,
@@ -487,13 +487,13 @@ bool launch_flash_f32(const FlashProblem &p, hipStream_t st, const FlashScratch 
         a.qw = p.rq.w;
         a.eps = p.rq.eps;
         const FlashPlan pl = flash_plan(BH, p.S_q, p.S_kv, p.D, kTimesF32, p.causal, scr);
-        FlashDeal deal;
-        a.split = flash_split_args(pl, BH, p.S_q, scr, deal);
+        FlashShares shares;
+        a.split = flash_split_args(pl, BH, p.S_q, scr, shares);
         if (!(pl.waves == 4 ? launch_d128<4>(a, FlashWhole{}, BH, st)
-              : pl.u > 0    ? launch_d128<8>(a, deal, BH, st)
+              : pl.u > 0    ? launch_d128<8>(a, shares, BH, st)
                             : launch_d128<8>(a, FlashWhole{}, BH, st)))
             return false;
-        return (a.split.n == 1 && a.split.u == 0) || launch_flash_combine(p, a.split, st);
+        return launch_flash_combine(p, a.split, shares.tail, st);
     }
     if (p.D > 1024)
         return fail("flash_f32: head dim " + std::to_string(p.D) + " > 1024 is not supported");

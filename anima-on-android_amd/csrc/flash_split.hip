@@ -11,6 +11,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace anima_hip {
 namespace {
@@ -22,17 +23,23 @@ constexpr int kD = kFlashD, kBM8 = kFlashRows8;
 struct CombineArgs {
     float *o;
     int64_t ob, oh, os;
-    int H, S_q, n_qtiles;
+    int H, S_q;
     FlashSplitArgs sa;
     TermOut ot;     // set: O as bf16 terms instead of f32 at o
     int64_t total;  // rows * 32 float4 columns
 };
 
-// One thread per (row, float4 of the head dim).  BAL: the rows are those of a
-// balanced grid's tail tiles, whose parts differ in number.  Bound by the
+// A balanced grid's tail tiles, and the query tiles of a (batch, head).
+struct CombineTail {
+    FlashTail t;
+    int n_qtiles;
+};
+
+// One thread per (row, float4 of the head dim).  Tail = CombineTail: the rows are
+// those of a balanced grid's tail tiles, whose parts differ in number.  Bound by the
 // partials' bytes (2304 tokens, B = 2, H = 16: 256 parts of 128 KiB).
-template <bool BAL>
-__global__ __launch_bounds__(256) void flash_combine_kernel(CombineArgs a)
+template <typename Tail>
+__global__ __launch_bounds__(256) void flash_combine_kernel(CombineArgs a, Tail tail)
 {
     const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
     if (idx >= a.total)
@@ -42,13 +49,13 @@ __global__ __launch_bounds__(256) void flash_combine_kernel(CombineArgs a)
     // Part s of this row is at partial row row0 + s * plane.
     int64_t bh, row0, plane;
     int q, n;
-    if (BAL) {
+    if constexpr (std::is_same<Tail, CombineTail>::value) {
         const int t = int(row / kBM8), r = int(row - int64_t(t) * kBM8);
-        const int tile = a.sa.full + t;
-        bh = tile / a.n_qtiles;
-        q = int(tile - bh * a.n_qtiles) * kBM8 + r;
-        const int64_t k0 = int64_t(t) * a.sa.nk;
-        const int g0 = int(k0 / a.sa.u), g1 = int((k0 + a.sa.nk - 1) / a.sa.u);
+        const int tile = tail.t.full + t;
+        bh = tile / tail.n_qtiles;
+        q = int(tile - bh * tail.n_qtiles) * kBM8 + r;
+        const int64_t k0 = int64_t(t) * tail.t.nk;
+        const int g0 = int(k0 / tail.t.u), g1 = int((k0 + tail.t.nk - 1) / tail.t.u);
         n = g1 - g0 + 1;
         if (q >= a.S_q)
             return;
@@ -118,17 +125,18 @@ bool term_out_ok(const TermOut &t)
 }
 
 FlashSplitArgs flash_split_args(const FlashPlan &pl, int64_t BH, int S_q, const FlashScratch &s,
-                                FlashDeal &deal)
+                                FlashShares &sh)
 {
     FlashSplitArgs sa;
     sa.BH = BH;
     size_t rows = 0;
     if (pl.u > 0) {
-        sa.full = pl.full;
-        sa.ntail = pl.ntail;
-        sa.nk = pl.nk;
-        sa.u = pl.u;
-        deal_pieces(pl.ntail, pl.nk, pl.u, deal, sa.ng, sa.nshorter);
+        FlashTail &t = sh.tail;
+        t.full = pl.full;
+        t.ntail = pl.ntail;
+        t.nk = pl.nk;
+        t.u = pl.u;
+        deal_pieces(pl.ntail, pl.nk, pl.u, sh.deal, t.ng, t.nshorter);
         sa.part = static_cast<float *>(s.balance);
         rows = pl.bytes / kFlashSlotBytes * kBM8;
     } else if (pl.splits > 1) {
@@ -142,15 +150,22 @@ FlashSplitArgs flash_split_args(const FlashPlan &pl, int64_t BH, int S_q, const 
     return sa;
 }
 
-int64_t flash_blocks(const FlashSplitArgs &sa, int64_t BH, int S_q, int BM)
+int64_t flash_blocks(const FlashSplitArgs &sa, const FlashWhole &, int64_t BH, int S_q, int BM)
 {
-    if (sa.u > 0)
-        return sa.full + sa.ng + sa.nshorter;
     return BH * flash_ceil_div(S_q, BM) * sa.n;
 }
 
-bool launch_flash_combine(const FlashProblem &p, const FlashSplitArgs &sa, hipStream_t st)
+int64_t flash_blocks(const FlashSplitArgs &, const FlashShares &sh, int64_t, int, int)
 {
+    return sh.tail.full + sh.tail.ng + sh.tail.nshorter;
+}
+
+bool launch_flash_combine(const FlashProblem &p, const FlashSplitArgs &sa, const FlashTail &tail,
+                          hipStream_t st)
+{
+    const bool bal = tail.u > 0;
+    if (sa.n == 1 && !bal)
+        return true;
     CombineArgs a;
     a.o = p.o;
     a.ob = p.os.b;
@@ -158,18 +173,18 @@ bool launch_flash_combine(const FlashProblem &p, const FlashSplitArgs &sa, hipSt
     a.os = p.os.s;
     a.H = p.H;
     a.S_q = p.S_q;
-    a.n_qtiles = int(flash_ceil_div(p.S_q, kBM8));
     a.sa = sa;
     a.ot = p.ot;
-    const bool bal = sa.u > 0;
-    a.total = (bal ? int64_t(sa.ntail) * kBM8 : sa.BH * p.S_q) * (kD / 4);
+    a.total = (bal ? int64_t(tail.ntail) * kBM8 : sa.BH * p.S_q) * (kD / 4);
     const int64_t nblk = flash_ceil_div(a.total, 256);
     if (nblk > INT32_MAX)
         return fail("flash_combine: problem too large for one launch");
     if (bal)
-        hipLaunchKernelGGL(flash_combine_kernel<true>, dim3(unsigned(nblk)), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(flash_combine_kernel<CombineTail>, dim3(unsigned(nblk)), dim3(256), 0,
+                           st, a, CombineTail{tail, int(flash_ceil_div(p.S_q, kBM8))});
     else
-        hipLaunchKernelGGL(flash_combine_kernel<false>, dim3(unsigned(nblk)), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(flash_combine_kernel<FlashWhole>, dim3(unsigned(nblk)), dim3(256), 0, st,
+                           a, FlashWhole{});
     return hip_ok(hipGetLastError(), "flash_combine_kernel launch");
 }
 

@@ -270,25 +270,26 @@ struct FlashWork {
         jn = sa.tiles;
         prow = sa.n > 1 ? (int64_t(sp) * sa.BH + bh) * S_q + int64_t(qt) * BM : -1;
     }
-    __device__ __forceinline__ FlashWork(const FlashSplitArgs &sa, const FlashDeal &deal,
+    __device__ __forceinline__ FlashWork(const FlashSplitArgs &, const FlashShares &sh,
                                          int n_qtiles, int, int BM)
     {
-        if (int(blockIdx.x) < sa.full) {
-            const int blk = xcd_major(blockIdx.x, sa.full);
+        const FlashTail &ta = sh.tail;
+        if (int(blockIdx.x) < ta.full) {
+            const int blk = xcd_major(blockIdx.x, ta.full);
             qt = blk % n_qtiles;
             bh = blk / n_qtiles;
             j0 = 0;
-            jn = sa.nk;
+            jn = ta.nk;
             prow = -1;
             return;
         }
-        // sa.full is a multiple of 256, so the pieces start at XCD 0.
-        const FlashPiece p = flash_piece(int(blockIdx.x) - sa.full, sa.ntail, sa.nk, sa.u, sa.ng,
-                                         deal);
+        // ta.full is a multiple of 256, so the pieces start at XCD 0.
+        const FlashPiece p = flash_piece(int(blockIdx.x) - ta.full, ta.ntail, ta.nk, ta.u, ta.ng,
+                                         sh.deal);
         j0 = p.j0;
         jn = p.jn;
-        qt = (sa.full + p.t) % n_qtiles;
-        bh = (sa.full + p.t) / n_qtiles;
+        qt = (ta.full + p.t) % n_qtiles;
+        bh = (ta.full + p.t) / n_qtiles;
         prow = int64_t(p.t + p.g) * BM;
     }
 };

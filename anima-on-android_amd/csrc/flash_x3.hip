@@ -447,7 +447,7 @@ bool launch_d128(const X3Args &a, const Deal &deal, int64_t BH, hipStream_t st)
     constexpr int BM = NW * 32;
     X3Args g = a;
     g.n_qtiles = (g.S_q + BM - 1) / BM;
-    const int64_t nblk = flash_blocks(g.split, BH, g.S_q, BM);
+    const int64_t nblk = flash_blocks(g.split, deal, BH, g.S_q, BM);
     if (nblk > INT32_MAX)
         return fail("flash_x3: problem too large for one launch");
     hipLaunchKernelGGL((flash_x3_d128<NW, Deal>), dim3(unsigned(nblk)), dim3(NW * 64), 0, st, g, deal);
@@ -525,13 +525,13 @@ bool launch_flash_x3(const FlashProblem &p, hipStream_t st, const FlashScratch &
         return launch_flash_keys(p, 2, a.dma32 != 0, st);
     if (p.rq.parts > 1)
         return fail("flash_x3: this launch shape takes no query planes");
-    FlashDeal deal;
-    a.split = flash_split_args(pl, BH, p.S_q, scr, deal);
+    FlashShares shares;
+    a.split = flash_split_args(pl, BH, p.S_q, scr, shares);
     if (!(pl.waves == 4 ? launch_d128<4>(a, FlashWhole{}, BH, st)
-          : pl.u > 0    ? launch_d128<8>(a, deal, BH, st)
+          : pl.u > 0    ? launch_d128<8>(a, shares, BH, st)
                         : launch_d128<8>(a, FlashWhole{}, BH, st)))
         return false;
-    return (a.split.n == 1 && a.split.u == 0) || launch_flash_combine(p, a.split, st);
+    return launch_flash_combine(p, a.split, shares.tail, st);
 }
 
 bool launch_vt_pack_terms(const float *v, Strides vs, uint16_t *vt, Strides vts, int B, int H,
