@@ -53,7 +53,7 @@ struct KeysArgs {
     float c;    // scale * log2(e), > 0
     int dma32;  // K/V^T tile rows fit 32-bit byte offsets from the tile start
     TermOut ot;
-    const float *qx, *qw, *qf;  // raw query rows (RawQ) in place of q when qx is set
+    const float *qx, *qw;  // raw query rows (RawQ, no RoPE) in place of q when qx is set
     int64_t rqb, rqh, rqs, qplane;
     int qparts;
     float eps;
@@ -66,14 +66,13 @@ __device__ __forceinline__ bool is_nan(float x) { return (__float_as_uint(x) << 
 
 // The terms of the workgroup's 64 raw rows, bit for bit those of the row prologue
 // (prologue.hip) and q_terms_from_raw: one lane per row adds the squares in
-// index order, every thread then scales, rotates and splits its own four
-// float4 (row tid / 32 + 16 i, columns 4 (tid % 32)), and the waves read their
-// fragments back.  q_terms_from_raw in every wave did the work of a row four
-// times over in some 1500 instructions run once, most of their time spent
-// fetching them: 18.7k of the 52k cycles of 256 x 512 f32x3, KQT here.
+// index order, every thread then scales and splits its own four float4 (row
+// tid / 32 + 16 i, columns 4 (tid % 32)), and the waves read their fragments
+// back.  (q_terms_from_raw in every wave would do the work of a row four times
+// over, once for each key group.)
 template <int TERMS>
 __device__ __forceinline__ void keys_q_terms(const KeysArgs &a, float *rows, const f32x4 (&v)[4],
-                                             int q0, int tid, bf16x8 (&qh)[8], bf16x8 (&ql)[8])
+                                             int tid, bf16x8 (&qh)[8], bf16x8 (&ql)[8])
 {
 #pragma clang fp contract(off)
     constexpr int kTermPitch = TERMS * kD + 8;  // 16-bit elements, 16 bytes against conflicts
@@ -91,7 +90,7 @@ __device__ __forceinline__ void keys_q_terms(const KeysArgs &a, float *rows, con
         }
         inv[tid] = inv_rms(ss, kD, a.eps);
     }
-    const int c4 = tid & 31, p0 = 4 * (c4 & 15);
+    const int c4 = tid & 31;
     f32x4 w = f32x4{1.f, 1.f, 1.f, 1.f};
     if (a.qw)
         w = *reinterpret_cast<const f32x4 *>(a.qw + 4 * c4);
@@ -103,19 +102,6 @@ __device__ __forceinline__ void keys_q_terms(const KeysArgs &a, float *rows, con
         f32x4 y = v[i] * inv[r];
         if (a.qw)
             y = y * w;
-        if (a.qf) {
-            // Pairs (p, p + 64): the other half's values are 16 lanes away.
-            const bool hi = c4 >= 16;
-            const float *fq =
-                a.qf + int64_t(min(q0 + r, a.S_q - 1)) * (2 * kD) + 4 * p0 + (hi ? 2 : 0);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float2 c = *reinterpret_cast<const float2 *>(fq + 4 * e);
-                const float other = __shfl_xor(y[e], 16);
-                const float ya = hi ? other : y[e], yb = hi ? y[e] : other;
-                y[e] = c.x * ya + c.y * yb;
-            }
-        }
         uint2 th, tl;
         split_terms4(y, th, tl);
         *reinterpret_cast<uint2 *>(terms + r * kTermPitch + 4 * c4) = th;
@@ -262,7 +248,7 @@ __global__ __launch_bounds__(512, 1) void flash_keys_d128(KeysArgs a)
             *reinterpret_cast<f32x4 *>(rows + (f >> 5) * kPitch + 4 * (f & 31)) = v[i];
         }
         __syncthreads();
-        keys_q_terms<TERMS>(a, rows, v, q0, tid, qh, ql);
+        keys_q_terms<TERMS>(a, rows, v, tid, qh, ql);
     } else {
         const u16 *qr = a.q + b * a.qb + h * a.qh + int64_t(min(qrow, a.S_q - 1)) * a.qs;
         const bf16x8 *src = reinterpret_cast<const bf16x8 *>(qr + 64 * half);
@@ -429,6 +415,8 @@ __global__ __launch_bounds__(512, 1) void flash_keys_d128(KeysArgs a)
 
 bool launch_flash_keys(const FlashProblem &p, int terms, bool dma32, hipStream_t st)
 {
+    if (p.rq.freqs)
+        return fail("flash_keys: raw query rows with RoPE are not taken");
     const int64_t BH = int64_t(p.B) * p.H;
     KeysArgs a;
     a.q = static_cast<const u16 *>(p.q);
@@ -448,7 +436,6 @@ bool launch_flash_keys(const FlashProblem &p, int terms, bool dma32, hipStream_t
     a.ot = p.ot;
     a.qx = p.rq.x;
     a.qw = p.rq.w;
-    a.qf = p.rq.freqs;
     a.rqb = p.rq.s.b; a.rqh = p.rq.s.h; a.rqs = p.rq.s.s;
     a.qparts = p.rq.parts;
     a.qplane = p.rq.plane;
