@@ -55,6 +55,7 @@ struct GemmArgs {
     int M, N;
     int tiles_m, tiles_n, splits;
     int chunks;          // K chunks per split
+    int m_first;         // tile order: the M tiles of an N tile are consecutive
 };
 
 // s_waitcnt vmcnt(n) for n < 64 (the count's high bits live in bits 15:14).
@@ -99,17 +100,14 @@ __global__ __launch_bounds__(kGemmWaves * 64, 1) void gemm_bf16_kernel(GemmArgs 
     const int col = lane & 31, half = lane >> 5;
     const int wm = wave & 1, wn = (wave >> 1) & 1, ks = wave >> 2;
 
-    // Tile order: consecutive ids (one XCD) share the split and the A rows.  The
-    // other way round (the M tiles of one N tile consecutive, near-square blocks
-    // of tiles per XCD) whole f32x3 calls took, with weights from HBM, 192 x 2048 x
-    // 1024 17.7 against 16.6 us so, 640 x 2048 x 2048 28.2 against 26.5, 512 x 6144
-    // x 2048 35.9 against 34.7, 640 x 8192 x 2048 68.3 against 63.6; at K = 8192
-    // and up to 512 rows the two are even within 1 %.
+    // Tile order: an XCD's consecutive ids take the N tiles of one M tile (and its A
+    // rows), or the M tiles (at most 8) of one N tile (launch_parts).
     const int blk = xcd_major_block();
-    const int tn = blk % g.tiles_n;
-    const int rest = blk / g.tiles_n;
-    const int tm = rest % g.tiles_m;
-    const int sp = rest / g.tiles_m;
+    const int fast = g.m_first ? g.tiles_m : g.tiles_n;
+    const int slow = g.m_first ? g.tiles_n : g.tiles_m;
+    const int rest = blk / fast, at = blk - rest * fast;
+    const int sp = rest / slow, row = rest - sp * slow;
+    const int tm = g.m_first ? at : row, tn = g.m_first ? row : at;
     const int row0 = tm * BM, col0 = tn * BN;
     const int total = g.chunks;
 
@@ -351,6 +349,14 @@ bool launch_parts(const uint16_t *a0, const uint16_t *a1, int64_t lda, const uin
     g.tiles_n = p.tiles_n;
     g.splits = p.splits;
     g.chunks = p.chunks;
+    // The M tiles first on [hi | lo] rows of four tiles and more.  The DiT's sampler
+    // step on such rows, two steps of 512 rows f32x3: 13.60 ms so, 13.78 the other way;
+    // 792 rows 19.64 and 19.82; even at 128 to 360 rows.  On two planes the other
+    // way is the better one, whole calls with weights from HBM: 192 x 2048 x 1024 17.7
+    // so, 16.6 the other way; 640 x 2048 x 2048 28.2 and 26.5; 512 x 6144 x 2048 35.9
+    // and 34.7; 640 x 8192 x 2048 68.3 and 63.6.  One term of K = 8192: 512 rows 34.8
+    // and 35.2, 640 49.9 and 46.6, 1024 55.7 and 53.3; even up to 384.
+    g.m_first = a1 ? a1 > a0 && a1 - a0 < lda && p.tiles_m >= 4 : p.tiles_m == 4;
     g.out = out;
     g.ldo = ldo;
     const int nblk = p.tiles_m * p.tiles_n * p.splits;
