@@ -408,7 +408,11 @@ bool run_attention_block(const BlockProblem &p, void *scratch, size_t scratch_by
     // the two-plane kernel took 288 us in six rounds of tiles that fill 1.1
     // each), which can write the attention's prepared operands in place of q,
     // k and v (H even, S a multiple of 64; the prologue pass, 48 us there, goes
-    // away).  Otherwise bf16 terms of x_m and a product each.
+    // away).  Otherwise, and where that is predicted to be 4 % faster, bf16 terms
+    // of x_m and a product each.  Sub-layers f32x3 as one grid and as three
+    // products: 4096 tokens of width 2048 455 and 444 us, 3072 387 and 381, 2048 of
+    // width 4096 642 and 580; 2816 of 2048 376 and 386, 4224 493 and 602, 8192 1132
+    // and 1179.
     AttnInputs in;
     const uint16_t *const w3[3] = {p.wq, p.wk, p.wv};
     const float *xm = reinterpret_cast<const float *>(hi);
@@ -426,8 +430,14 @@ bool run_attention_block(const BlockProblem &p, void *scratch, size_t scratch_by
         qp.H = H;
         qp.eps = p.eps;
         qp.mode = p.mode;
-        prep = D == 128 && gemm_f32a_qkv_supported(xm, Dm, w3, Dm, Dm, qp);
-        three = prep || (M <= INT32_MAX &&
+        // What the epilogue adds, exposed in the last round of tiles; the prologue pass.
+        constexpr double kQkvEpilogueUs = 18.0, kPrologueBytesPerUs = 4.5e6;
+        const double grid = M <= INT32_MAX / 3 ? gemm_f32a_wide_us(int(M), 3 * HD, Dm) : 0.0;
+        const double each = M <= INT32_MAX ? 3.0 * linear_terms_us(int(M), HD, Dm) : 0.0;
+        const double prologue = 24.0 * double(M) * HD / kPrologueBytesPerUs;
+        prep = D == 128 && gemm_f32a_qkv_supported(xm, Dm, w3, Dm, Dm, qp) &&
+               grid + kQkvEpilogueUs <= 1.04 * (each + prologue);
+        three = prep || (M <= INT32_MAX && grid <= 1.04 * each &&
                          gemm_f32a_three_supported(int(M), HD, Dm, Dm, Dm, HD, xm, w3, q));
     }
     if (!launch_ln_modulate(p.x, Dm, p.mod, 3 * int64_t(Dm), three ? nullptr : hi,
@@ -476,9 +486,14 @@ bool run_attention_block(const BlockProblem &p, void *scratch, size_t scratch_by
     // them (lo_t = the hi block's size).  Other head dims, a shape the
     // library GEMM does not take (launch_linear's exact f32 fallback needs
     // O itself), or one that the f32-activation kernel runs better than the
-    // kernels on terms (4608 rows: 75 against 96 us): f32 O at o.
+    // kernels on terms (4608 rows: 75 against 96 us): f32 O at o.  Its epilogue
+    // saves half of the residual pass; widths below 1024 stay on terms (512, 4
+    // heads: 3 to 6 % slower up to 3072 rows, 1 % faster from 4608).
     const bool lib = linear_terms_supported(int(M), Dm, HD, p.wo, HD, y, Dm);
-    const bool f32a_out = !bf16 && linear_takes_f32a(o, HD, p.wo, HD, y, Dm, int(M), Dm, HD);
+    const double residual = 6.0 * double(M) * Dm / 4.5e6;
+    const bool f32a_out =
+        !bf16 && lib && Dm >= 1024 && gemm_f32a_fits(int(M), Dm, HD, HD, HD, Dm, o, p.wo, y) &&
+        1.04 * gemm_f32a_us(int(M), Dm, HD) <= linear_terms_us(int(M), Dm, HD) + residual;
     const bool terms_out = D == 128 && !f32a_out && lib;
     const int64_t kp = linear_terms_ld(HD);
     const size_t hi_bytes = round_up256(size_t(M) * size_t(kp) * 2);
@@ -507,7 +522,7 @@ bool run_attention_block(const BlockProblem &p, void *scratch, size_t scratch_by
                                                   3 * int64_t(Dm), B, S, Dm, HD, st)
                    : launch_linear_residual(o, HD, p.wo, HD, p.x, Dm, p.mod + 2 * int64_t(Dm),
                                             3 * int64_t(Dm), B, S, Dm, HD, lin, s.lin, st);
-    if (f32a_out && lib && S >= 32)
+    if (f32a_out && S >= 32)
         return launch_gemm_f32a_residual(o, HD, p.wo, HD, p.x, Dm, p.mod + 2 * int64_t(Dm),
                                          3 * int64_t(Dm), S, int(M), Dm, HD, st);
     const size_t terms_bytes = hi_bytes * (bf16 ? 1 : 2);

@@ -167,6 +167,7 @@ bool launch_linear(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, 
 // launch_linear (exact) runs this shape on gemm_f32a.hip.
 bool linear_takes_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, const float *c,
                        int64_t ldc, int M, int N, int K);
+double linear_terms_us(int M, int N, int K);
 
 // A split into [hi | lo] rows of 2*linear_terms_ld(K) bf16 (the product with
 // a weight whose rows are [W | W], K' = 2 * linear_terms_ld(K), is then one
@@ -202,12 +203,13 @@ bool launch_gemm_large_f32a(const float *a, int64_t lda, const uint16_t *w, int6
 // terms C is bit-identical to the split pass plus launch_gemm_large on the
 // term rows.  gemm_f32a_fits: shapes and alignments it takes;
 // gemm_f32a_supported: and at least 256 tiles of 256 x 256; gemm_f32a_us: the
-// two-term product's predicted time.
+// two-term product's predicted time, gemm_f32a_wide_us: that in 256 x 256 tiles.
 bool gemm_f32a_fits(int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc, const float *a,
                     const void *w, const void *c);
 bool gemm_f32a_supported(int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc,
                          const float *a, const void *w, const void *c);
 double gemm_f32a_us(int M, int N, int K);
+double gemm_f32a_wide_us(int M, int N, int K);
 bool launch_gemm_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, float *c,
                       int64_t ldc, int M, int N, int K, bool two_terms, hipStream_t st);
 // x [M][ldx] += gate[m / S] * (a W^T), the two-term product as launch_gemm_f32a's

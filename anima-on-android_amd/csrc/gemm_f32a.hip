@@ -545,6 +545,12 @@ double gemm_f32a_us(int M, int N, int K)
     return 5.0 + (us - 5.0) * K / 2048;
 }
 
+double gemm_f32a_wide_us(int M, int N, int K)
+{
+    const double us = tiles_us((int64_t(M) + kFaBM - 1) / kFaBM, N, kFaNB);
+    return 5.0 + (us - 5.0) * K / 2048;
+}
+
 // Shapes the kernel takes: K a multiple of 32, 16-byte aligned A and W rows,
 // byte offsets of a tile's rows within 32 bits.
 bool gemm_f32a_fits(int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc, const float *a,

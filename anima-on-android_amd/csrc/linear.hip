@@ -338,6 +338,20 @@ bool linear_takes_f32a(const float *a, int64_t lda, const uint16_t *w, int64_t l
     return 1.04 * gemm_f32a_us(M, N, K) <= other;
 }
 
+// The same for launch_linear_terms' two-term product (its kernel in 128 x 256 tiles
+// 51 a round at K = 2048, a last round of at least 36; two library products 15 us,
+// the rest as above).
+double linear_terms_us(int M, int N, int K)
+{
+    const int64_t tiles = ((int64_t(M) + 127) / 128) * ((int64_t(N) + 255) / 256);
+    if (tiles < 256)
+        return 15.0 + (4.0 * M * double(N) / 1.15e9 + 0.002) * K;
+    const int64_t rest = tiles % 256;
+    const double us =
+        double(tiles / 256) * 51.0 + (rest ? std::max(36.0, 0.22 * double(rest)) : 0.0);
+    return 4.0 + (us - 4.0) * K / 2048;
+}
+
 bool launch_linear(const float *a, int64_t lda, const uint16_t *w, int64_t ldw, float *c,
                    int64_t ldc, int M, int N, int K, bool exact, void *scratch,
                    size_t scratch_bytes, hipStream_t st)

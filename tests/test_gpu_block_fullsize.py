@@ -88,11 +88,12 @@ def test_cross_attention_block_4096(mode):
     _check(out, ref, x, mode)
 
 
-# The three projections as one grid (11 x 24 tiles of 256 x 256), which writes the
-# attention's prepared operands (S a multiple of 64; two batch entries whose
-# boundary falls inside a tile) or q, k and v (S ragged).
+# The three projections as one grid (11 x 24 and 14 x 24 tiles of 256 x 256), which
+# writes the attention's prepared operands (S a multiple of 64; two batch entries
+# whose boundary falls inside a tile) or, at 3355 tokens, q, k and v (S ragged); 2601
+# tokens run three products.
 @pytest.mark.parametrize("mode", [rt.F32, rt.F32X3])
-@pytest.mark.parametrize("b,grid", [(2, (44, 32)), (1, (51, 51))])
+@pytest.mark.parametrize("b,grid", [(2, (44, 32)), (1, (51, 51)), (1, (55, 61))])
 def test_self_attention_block_one_projection_grid(mode, b, grid):
     _, x, mod, w, qw, kw = _inputs(4403 + b, b, grid[0] * grid[1])
     ref = fullsize.block_ref(x, mod, *w, qw, kw, oracle.rope_freqs(*grid), None)
