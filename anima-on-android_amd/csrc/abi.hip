@@ -738,12 +738,16 @@ bool sdpa_heads(Runtime &r, int64_t h0, int nh, int S_q, int S_kv, int D, float 
 // Head groups of a host-pointer SDPA: when the copies are large, the most
 // groups (4 or 2) that still fill the GPU each, or two where the whole call does
 // not fill it either (its kernels share out the keys of each query tile, and
-// the groups' do the same); else one.  Group g+1 uploads while group g computes,
+// the groups' do the same) and the output, whose first half then comes back
+// while the rest uploads, is at least a twelfth of the copies; else one.  Group g+1 uploads while group g computes,
 // and group g's output comes back while later groups upload.  In that last
 // case two groups against one ran 1.91 against 2.32 ms (BH = 32, S = 1024), 1.97
 // against 2.42 (16, 2048) and 2.12 against 2.79 (8, 4096); four 2.30, 2.28 and
 // 2.54, each group's copies paying their own latencies; at 50 MB of copies two
-// were 2 % faster, at 34 MB 8 to 12 % slower.
+// were 2 % faster, at 34 MB 8 to 12 % slower.  By the output's share (16 heads,
+// f32): 1536 queries on 3072 keys (0.17) 1.98 against 2.48 ms, 1024 on 4096 (0.1)
+// 2.20 against 2.31, 512 on 4096 (0.06) 2.15 against 1.89, 512 on 8192 3.79 against
+// 3.37.
 int sdpa_groups(int BH, int S_q, int S_kv, int D)
 {
     const int64_t bytes = int64_t(BH) * (2 * int64_t(S_q) + 2 * int64_t(S_kv)) * D * 4;
@@ -755,7 +759,8 @@ int sdpa_groups(int BH, int S_q, int S_kv, int D)
         if (flash_fills_gpu(BH / G, S_q, D))
             return G;
     }
-    return !flash_fills_gpu(BH, S_q, D) && BH % 2 == 0 ? 2 : 1;
+    const int64_t out = int64_t(BH) * S_q * D * 4;
+    return !flash_fills_gpu(BH, S_q, D) && BH % 2 == 0 && 12 * out >= bytes ? 2 : 1;
 }
 
 // Shared body of the host-pointer SDPA entries ([BH, S, D] f32 host arrays).
