@@ -118,10 +118,13 @@ inline FlashPlan split_plan(int64_t BH, int S_q, int S_kv, int D)
 // workgroups.  One more round is as short as the last split, where each engine's
 // (8 CUs) extra workgroups are fewer than its workgroups of that split, which end
 // first (T4 = 96 on 5 key tiles, three splits of 2, 2 and 1, f32: 3 tiles' time).
-inline double split_tiles(const FlashPlan &sp, int64_t T4, int64_t n)
+inline double split_tiles(const FlashPlan &sp, int64_t T4, int64_t n, bool causal)
 {
     constexpr int64_t kEngines = 32;
-    const int64_t blocks = T4 * sp.splits, extra = blocks - kFlashTargetBlocks;
+    // Causal: a split beyond its queries ends at once, about (splits - 1) / 2 of them
+    // (7 heads of 2500, f32, two splits: call 1359 us, 4-wave workgroups 1450).
+    const int64_t blocks = causal ? T4 * (sp.splits + 1) / 2 : T4 * sp.splits;
+    const int64_t extra = blocks - kFlashTargetBlocks;
     const int64_t whole = flash_ceil_div(blocks, kFlashTargetBlocks) * sp.tiles;
     if (extra <= 0 || flash_ceil_div(extra, kEngines) >= 8 / sp.splits)
         return double(whole);
@@ -181,7 +184,7 @@ inline FlashPlan flash_plan(int64_t BH, int S_q, int S_kv, int D, const FlashTim
         consider(small, rounds(T4) * n * t.w4);
         const FlashPlan sp = split_plan(BH, S_q, S_kv, D);
         if (sp.splits > 1 && sp.bytes <= s.part_bytes)
-            consider(sp, split_tiles(sp, T4, int64_t(n)) * t.w4 + t.split +
+            consider(sp, split_tiles(sp, T4, int64_t(n), causal) * t.w4 + t.split +
                              t.split_mb * 1e-6 * double(sp.bytes));
     }
     const FlashPlan bal = balanced_plan(BH, S_q, S_kv, D);

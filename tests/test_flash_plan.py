@@ -58,6 +58,14 @@ def test_measured_shapes(shape, mode, BH, S_q, S_kv, fastest):
     assert shape(mode, BH, S_q, S_kv) == fastest
 
 
+@pytest.mark.parametrize("mode,BH,S", [(rt.F32, 7, 2500), (rt.F32, 20, 1000), (rt.BF16, 9, 2000),
+                                       (rt.F32X3, 7, 2500)])
+def test_causal_split(shape, mode, BH, S):
+    """Causal splits of which a third ends at once and the rest fills one round
+    (f32: host calls 1376 against 1530 us whole, 1343 against 1414)."""
+    assert shape(mode, BH, S, S, causal=True, keys=False) == "split"
+
+
 @pytest.mark.parametrize("mode,B,H,S_q,S_kv", test_gpu_keys.CASES)
 def test_keys_cases(shape, mode, B, H, S_q, S_kv):
     assert shape(mode, B * H, S_q, S_kv) == "keys"
