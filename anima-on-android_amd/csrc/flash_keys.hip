@@ -14,17 +14,16 @@
 // (keys): wave (r, g) takes rows 32r .. 32r+31 and key tiles g, g + 4, ..., with
 // its own running max, sum and O; the four parts of a row are merged through
 // LDS at the end.  Four times the workgroups, two waves per SIMD, no second
-// launch; each K/V tile serves 64 rows instead of 128 or 256, so the kernel is
-// bound by the L2 -> LDS stream (128 KiB per round of four tiles, about 35 bytes
-// per clock and CU) where the grid fills the GPU.
+// launch; each K/V tile serves 64 rows instead of 128 or 256.  Bound by the chain
+// of a round, whose copies, products and softmax follow one another between two
+// barriers: on its fullest grid (1024 x 1024, 16 heads, f32x3) the MFMA pipes are
+// busy 26 % of the cycles and LDS 11 %, waves wait 36 %, and 12 MB come from HBM.
 // Whole attention calls on MI355X before and now, 16 heads (f32x3 / bf16): self
 // 256 tokens 24.7 -> 22.3 / 17.8 -> 15.5 us, 1024 tokens 50.4 -> 45.6 / 39.1 ->
 // 30.3; cached cross-attention, query rows normalised in here, 2 x 256 on 512
-// 28.8 -> 17.9 / 20.7 -> 12.0, 1024 x 512 34.5 -> 20.0 / 22.6 -> 12.7.  Cycles of
-// 2 x 256 tokens, self f32x3 (31.6k): 11.4k until the first K tiles and Q are
-// there, 2.1k to 2.4k a phase of MFMAs and 0.6k to 0.9k more for its copies
-// (waiting for K and V^T with a barrier of its own each, so that more copies are
-// in flight, was 3 to 16 % slower), 6.2k for the merge.
+// 28.8 -> 17.9 / 20.7 -> 12.0, 1024 x 512 34.5 -> 20.0 / 22.6 -> 12.7.  (Waiting
+// for K and V^T with a barrier of its own each, so that more copies are in
+// flight, was 3 to 16 % slower.)
 //
 // Per key group one K tile and one V^T tile (16 KiB each: 32 keys of terms, 64
 // of bf16), single-buffered and refilled in turn: V^T lands while the scores

@@ -105,18 +105,21 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g)
 }
 
 // C = A . W^T on f32 MFMA from DMA-staged tiles: 64 x 64 of C per workgroup, 4
-// waves in a 2x2 grid each owning 32 x 32.  Bound by the f32 MFMA pipe, which
-// takes 64 cycles per 32x32x2 product: a chunk of 32 k needs 16 bytes per clock
-// from L2 and 32 from LDS, inside what a CU gets (35 and 128), so the small tile
-// costs little and comes out more even over the CUs.  Two stages of one chunk
+// waves in a 2x2 grid each owning 32 x 32.  Bound by the f32 MFMA pipe (busy 83 %
+// of the cycles at 8192x2048x2048, 74 % at 2400x2048x2048, whose 1216 tiles are
+// less than the 1280 that five to a CU make), which takes 64 cycles per 32x32x2
+// product: a chunk of 32 k needs 16 bytes per clock from L2 and 32 from LDS,
+// inside what a CU gets (35 and 128), so the small tile costs little and comes
+// out more even over the CUs.  Two stages of one chunk
 // (32 KiB, five workgroups to a CU), one barrier per chunk; other workgroups'
 // products fill a wave's waits.  Two accumulators take the products of even and
 // odd k: shorter chains, and rounding errors 0.7 times one chain's.
 // Whole calls on MI355X, before (gemm_kernel) and now: 2400x2048x2048 785 ->
-// 187 us (108 TFLOP/s), 8192x2048x2048 1061 -> 537 (128), 512x2048x8192 2575 ->
-// 155, 100x2048x2048 365 -> 40.  Measured beside it at the first two shapes:
-// 128 x 128 tiles, two workgroups to a CU 257 / 518 us; three stages and three
-// workgroups 191 / 567; one accumulator 188 / 542; no raised priority 191 / 558.
+// 171 us (118 TFLOP/s; up to 187 by box and load), 8192x2048x2048 1061 -> 537
+// (128), 512x2048x8192 2575 -> 155, 100x2048x2048 365 -> 40.  Measured beside it
+// at the first two shapes in one run that gave it 187 / 537: 128 x 128 tiles, two
+// workgroups to a CU 257 / 518 us; three stages and three workgroups 191 / 567;
+// one accumulator 188 / 542; no raised priority 191 / 558.
 //
 // A chunk's row holds 32 k as eight 16-byte pieces; piece c of row r is at
 // c ^ ((r >> 1) & 7), so the 16 rows that a fragment read serves per clock fall
